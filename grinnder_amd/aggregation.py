@@ -338,7 +338,7 @@ class _GCNLinearAggregatePadded(torch.autograd.Function):
     def backward(ctx, gy: Tensor):
         from torch.nn.functional import pad
 
-        from grinnder_amd.dense import gemm_nt, gemm_tn
+        from grinnder_amd.dense import gemm_nt_split, gemm_tn
         x, wp = ctx.saved_tensors
         plan: DevicePlan = ctx.plan
         d, dp = ctx.d, wp.size(0)
@@ -350,7 +350,7 @@ class _GCNLinearAggregatePadded(torch.autograd.Function):
             dx = ctx.ln_sink.hand_over(dz, wp, ctx.x_shape)
         elif ctx.needs_input_grad[0]:
             with dense_region("dx", dz.size(0), dp, wp.size(1)):
-                dx = gemm_nt(dz, wp.t().contiguous())
+                dx = gemm_nt_split(dz, wp.t().contiguous())
         if ctx.needs_input_grad[1]:
             with dense_region("dw", dz.size(0), dp, x.size(1)):
                 dw = gemm_tn(dz, x)[:d]
@@ -533,8 +533,8 @@ class _GCNAggregateLNReLU(torch.autograd.Function):
                                                             bt, ctx.has_bias)
         else:
             if prod is not None:
-                from grinnder_amd.dense import gemm_nt
-                gout = gout + gemm_nt(prod[0], prod[1].t().contiguous())
+                from grinnder_amd.dense import gemm_nt_split
+                gout = gout + gemm_nt_split(prod[0], prod[1].t().contiguous())
             gh, dgamma, dbeta, db = ln_act_backward(gout, h, mean, rstd, g, bt, ctx.has_bias)
         dz = None
         if ctx.sink is not None:
@@ -1026,8 +1026,8 @@ class _GATAttentionLN(torch.autograd.Function):
                 rowdot=rowdot)
         else:
             if prod is not None:
-                from grinnder_amd.dense import gemm_nt
-                gout = gout + gemm_nt(prod[0], prod[1].t().contiguous())
+                from grinnder_amd.dense import gemm_nt_split
+                gout = gout + gemm_nt_split(prod[0], prod[1].t().contiguous())
             gh, dgamma, dbeta, db = ln_act_backward(gout, h, mean, rstd, g, bt, has_bias,
                                                     ctx.act, shift=ctx.bias, rowdot=rowdot)
         dhs, datt_src, datt_dst = _attention_backward(plan, hs, a_src, a_dst, s, d, m, den, gh,

@@ -1,23 +1,13 @@
-// Weight-gradient GEMM for the dense per-layer transform: C[M,N] = A^T B with
-// A [K, M] and B [K, N] row-major and K (the node count) in the millions,
-// M, N <= a few hundred.  fp32 on the gfx950 matrix cores
-// (v_mfma_f32_16x16x4_f32 or v_mfma_f32_32x32x2_f32), deterministic split-K.
-//
-// Workgroup tile 128 x 128 (4 wavefronts as 2 x 2 tiles of 64 x 64, each
-// 4 x 4 MFMA blocks of 16 x 16 or 2 x 2 of 32 x 32); K is walked in steps of
-// 16 rows staged in LDS,
-// with the next step's global loads issued before the current step's MFMAs.
-// Workgroup (tile t, chunk z) owns the K rows [z*kchunk, (z+1)*kchunk) and
-// writes its partial tile to part[z]; the partials are then summed over z in
-// order, so the result does not depend on scheduling.
-//
-// Workgroups are dispatched round-robin over the 8 XCDs (linear id mod 8), and
-// each XCD has its own L2.  The linear id is decoded so that the T output tiles
-// of one K chunk are consecutive workgroups of the same XCD: the A and B rows
-// of that chunk are fetched from HBM once and re-read from that XCD's L2.
+// Dense products of the per-layer transform on the gfx950 matrix cores: the
+// forward C = A B^T + bias on the fp32 matrix instructions (gr_gemm_nt, and
+// with a LayerNorm epilogue gr_linear_ln_act); the weight gradient C[M, N] =
+// A^T B over millions of rows (gr_gemm_tn) and the input gradient's row-block
+// product (gr_gemm_nt_split) on the bf16 ones, with operands split into three
+// pieces (bf16x3.h).
 #include <algorithm>
 #include <type_traits>
 
+#include "gemm_bf3.h"
 #include "gr_internal.h"
 #include "wave.h"
 
@@ -26,192 +16,72 @@ namespace gr_gemm {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-constexpr int TM = 128;
-constexpr int TN = 128;
-constexpr int TK = 16;
-constexpr int PAD = 16;  // LDS row padding: rows k and k+1 land 16 banks apart
+constexpr int kXcds = gr_bf3::kXcds;
 
-// Loads rows [k, k + TK) x columns [c0, c0 + W) of a row-major [K, ld] matrix
-// into registers: 16 * W floats per workgroup, W / 16 per thread (W = 128 or
-// 64).  Out-of-range elements read as 0.
-template <int VEC, int W>
-__device__ __forceinline__ void load_tile(const float* __restrict__ src, int64_t ld, int64_t k,
-                                          int64_t k_end, int c0, int cols,
-                                          float (&r)[W / 16]) {
-  const int tid = threadIdx.x;
-  if constexpr (VEC == 4) {
-    constexpr int Q = W / 4;  // float4 slots per row
-#pragma unroll
-    for (int i = 0; i < W / 64; ++i) {
-      const int idx = tid + i * 256;
-      const int row = idx / Q;
-      const int c = c0 + (idx % Q) * 4;
-      const int64_t kr = k + row;
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (kr < k_end && c < cols) v = *reinterpret_cast<const float4*>(src + kr * ld + c);
-      r[i * 4 + 0] = v.x;
-      r[i * 4 + 1] = v.y;
-      r[i * 4 + 2] = v.z;
-      r[i * 4 + 3] = v.w;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < W / 16; ++i) {
-      const int idx = tid + i * 256;
-      const int row = idx / W;
-      const int c = c0 + (idx % W);
-      const int64_t kr = k + row;
-      r[i] = (kr < k_end && c < cols) ? src[kr * ld + c] : 0.f;
-    }
-  }
-}
-
-template <int VEC, int W, int P = PAD>
-__device__ __forceinline__ void store_tile(float (*lds)[W + P], const float (&r)[W / 16]) {
-  const int tid = threadIdx.x;
-  if constexpr (VEC == 4) {
-    constexpr int Q = W / 4;
-#pragma unroll
-    for (int i = 0; i < W / 64; ++i) {
-      const int idx = tid + i * 256;
-      const int row = idx / Q;
-      const int c = (idx % Q) * 4;
-      *reinterpret_cast<float4*>(&lds[row][c]) =
-          make_float4(r[i * 4 + 0], r[i * 4 + 1], r[i * 4 + 2], r[i * 4 + 3]);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < W / 16; ++i) {
-      const int idx = tid + i * 256;
-      lds[idx / W][idx % W] = r[i];
-    }
-  }
-}
-
-constexpr int kXcds = 8;
-// Largest K the split-K weight-gradient product runs on 32 x 32 blocks with
-// 128-column tiles (64-column tiles always take them).  Measured on one box:
-// at K = 2.45M the 32 x 32 form is level at 256 x 256 and 10% faster at
-// 256 x 100 (11% for 64-column tiles, 48 x 256); at K = 10M it is 2-3%
-// slower (256 x 256 and 256 x 1024).
-constexpr int64_t kTn32MaxK = int64_t(1) << 22;
-
-// BN = 128, 64 or 32 output columns per workgroup (64 and 32 for narrow N;
-// 32 takes B with 4-byte loads).  BLK = 16: each wavefront's 64 x BN/2 tile
-// as 16 x 16 blocks of v_mfma_f32_16x16x4_f32; BLK = 32: as 32 x 32 blocks of
-// v_mfma_f32_32x32x2_f32 (BN 64 or 128), with rows of the LDS tiles 32 floats
-// apart mod 64 banks so the two k rows a 32x32x2 step reads fall on
-// distinct banks.
-template <int VA, int VB, int BN, int BLK = 16>
-__global__ __launch_bounds__(256) void gemm_tn_splitk(const float* __restrict__ A, int64_t lda,
-                                                      const float* __restrict__ B, int64_t ldb,
-                                                      int M, int N, int64_t K, int64_t kchunk,
-                                                      int nchunks, int tiles_m, int tiles,
-                                                      float* __restrict__ part) {
-  static_assert(BLK == 16 || (BLK == 32 && BN >= 64), "32 x 32 blocks need 64+ columns");
-  constexpr int P = BLK == 16 ? PAD : 32;
-  constexpr int MI = 64 / BLK;          // row blocks per wavefront
-  constexpr int NJ = BN / 2 / BLK;      // column blocks per wavefront
-  constexpr int KSTEP = 64 / BLK;       // k per MFMA: 4 or 2
-  typedef typename std::conditional<BLK == 16, floatx4, floatx16>::type accx;
-  __shared__ float As[TK][TM + P];
-  __shared__ float Bs[TK][BN + P];
-  const int w = blockIdx.x;
-  const int q = w / kXcds;
-  const int t = q % tiles;
-  const int z = (q / tiles) * kXcds + w % kXcds;
-  if (z >= nchunks) return;  // whole workgroup: no barrier is pending
-  const int m0 = (t % tiles_m) * TM;
-  const int n0 = (t / tiles_m) * BN;
-  const int64_t k_begin = (int64_t)z * kchunk;
-  const int64_t k_end = k_begin + kchunk < K ? k_begin + kchunk : K;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm = (wave & 1) * 64;
-  const int wn = (wave >> 1) * (BN / 2);
-  const int lr = lane % BLK;  // row (A) / column (B) inside a block
-  const int lk = lane / BLK;  // k inside an MFMA step
-
-  accx acc[MI][NJ];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[i][j] = accx{};
-
-  float ra[TM / 16], rb[BN / 16];
-  load_tile<VA, TM>(A, lda, k_begin, k_end, m0, M, ra);
-  load_tile<VB, BN>(B, ldb, k_begin, k_end, n0, N, rb);
-  for (int64_t k = k_begin; k < k_end; k += TK) {
-    __syncthreads();  // previous step's MFMA reads of the LDS tiles are done
-    store_tile<VA, TM, P>(As, ra);
-    store_tile<VB, BN, P>(Bs, rb);
-    __syncthreads();
-    if (k + TK < k_end) {
-      load_tile<VA, TM>(A, lda, k + TK, k_end, m0, M, ra);
-      load_tile<VB, BN>(B, ldb, k + TK, k_end, n0, N, rb);
-    }
-#pragma unroll
-    for (int kk = 0; kk < TK; kk += KSTEP) {
-      float a[MI], b[NJ];
-#pragma unroll
-      for (int i = 0; i < MI; ++i) a[i] = As[kk + lk][wm + i * BLK + lr];
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) b[j] = Bs[kk + lk][wn + j * BLK + lr];
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          if constexpr (BLK == 16)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
-          else
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-    }
-  }
-
-  // BLK = 16: lane holds column lr, rows 4 lk + r (r < 4).  BLK = 32: lane
-  // holds column lr, rows 8 (r / 4) + 4 lk + r % 4 (r < 16).
-  constexpr int RPL = BLK == 16 ? 4 : 16;
-  float* out = part + (int64_t)z * M * N;
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int n = n0 + wn + j * BLK + lr;
-#pragma unroll
-      for (int r = 0; r < RPL; ++r) {
-        const int row = BLK == 16 ? lk * 4 + r : (r / 4) * 8 + lk * 4 + r % 4;
-        const int m = m0 + wm + i * BLK + row;
-        if (m < M && n < N) out[(int64_t)m * N + n] = acc[i][j][r];
-      }
-    }
-}
-
-// C = sum_z part[z] in z order over the rows x cols partial tiles
-// (grid-stride).  With `trans` the partial holds C^T: element (r, q) goes to
-// c[q * rows + r].
-__global__ __launch_bounds__(256) void sum_partials(const float* __restrict__ part, int splits,
-                                                    int64_t rows, int64_t cols, float beta,
-                                                    int trans, float* __restrict__ c) {
+// C = sum_z part[z] over the rows x cols partial tiles.  With `trans` the
+// partial holds C^T: element (r, q) goes to c[q * rows + r].  A workgroup takes
+// 64 elements; wavefront w sums z = w, w + kSumWaves, ... in order, eight in
+// flight, and the wavefronts' sums are added in order, so the result does not
+// depend on scheduling.  The loads of one element are a serial chain only
+// within a wavefront: 512 partials of 256 x 48 take 8 us, against 35 us with
+// one thread an element.
+constexpr int kSumWaves = 8;
+__global__ __launch_bounds__(kSumWaves * 64) void sum_partials(
+    const float* __restrict__ part, int splits, int64_t rows, int64_t cols, float beta,
+    int trans, float* __restrict__ c) {
+  __shared__ float sums[kSumWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t elems = rows * cols;
-  const int64_t stride = (int64_t)gridDim.x * 256;
-  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < elems; e += stride) {
+  const int64_t stride = (int64_t)gridDim.x * 64;
+  for (int64_t e0 = (int64_t)blockIdx.x * 64; e0 < elems; e0 += stride) {
+    const int64_t e = e0 + lane < elems ? e0 + lane : elems - 1;
     float s = 0.f;
-    int z = 0;
-    for (; z + 4 <= splits; z += 4) {
-      const float a0 = part[(int64_t)(z + 0) * elems + e];
-      const float a1 = part[(int64_t)(z + 1) * elems + e];
-      const float a2 = part[(int64_t)(z + 2) * elems + e];
-      const float a3 = part[(int64_t)(z + 3) * elems + e];
-      s += a0;
-      s += a1;
-      s += a2;
-      s += a3;
+    int z = wave;
+    for (; z + 7 * kSumWaves < splits; z += 8 * kSumWaves) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = part[(int64_t)(z + u * kSumWaves) * elems + e];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += v[u];
     }
-    for (; z < splits; ++z) s += part[(int64_t)z * elems + e];
-    const int64_t d = trans ? (e % cols) * rows + e / cols : e;
-    c[d] = beta != 0.f ? fmaf(beta, c[d], s) : s;
+    for (; z < splits; z += kSumWaves) s += part[(int64_t)z * elems + e];
+    sums[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0 && e0 + lane < elems) {
+#pragma unroll
+      for (int w = 1; w < kSumWaves; ++w) s += sums[w][lane];
+      const int64_t d = trans ? (e % cols) * rows + e / cols : e;
+      c[d] = beta != 0.f ? fmaf(beta, c[d], s) : s;
+    }
+    __syncthreads();
   }
+}
+
+// A narrow product (m <= 64 < n) runs as C^T = B^T A, so the narrow side falls
+// on the tile's short side; the partials are summed into C with a transposed
+// store.
+inline bool tn_swaps(int64_t m, int64_t n) { return m <= 64 && n > 64; }
+
+// Tile of the split-K product (pm >= pn after the swap), by measurement (us;
+// m x n over k, without the sum of the partials):
+//   both sides past 128: 256 x 256, a workgroup per CU (256 x 256 over 1M
+//     rows 763, 128 x 128 936; 200 x 500 over 30k 50 and 56);
+//   else 128 x 128 (100 x 256 over 150k 68; 256 x 256 tiles 96);
+//   up to 64 columns: 256 x 64 (256 x 48 over 200k 59, 128 x 128 84);
+//   up to 32 columns: 128 x 32 (256 x 20 over 100k 28, 256 x 64 30);
+//   64 x 64 where K is too short for the larger tiles to fill the chip in
+//     chunks of 64 rows (64 x 128 over 10k rows 7.1, 128 x 64 10).
+struct TnTile {
+  int bm, bn, target;  // target: workgroups of the default split count
+};
+inline TnTile tn_tile(int64_t pm, int64_t pn, int64_t k) {
+  TnTile t = pn <= 32    ? TnTile{128, 32, 1024}
+             : pn <= 64  ? TnTile{256, 64, 512}
+             : pn <= 128 || pm <= 128 ? TnTile{128, 128, 512}
+                                      : TnTile{256, 256, 256};
+  const int64_t tiles = ((pm + t.bm - 1) / t.bm) * ((pn + t.bn - 1) / t.bn);
+  if (tiles * (k / 64) < 256) t = TnTile{64, 64, 512};
+  return t;
 }
 
 }  // namespace gr_gemm
@@ -221,12 +91,15 @@ extern "C" int gr_gemm_tn_workspace(int64_t m, int64_t n, int64_t k, int64_t* sp
   gr::clear_error();
   GR_REQUIRE(m >= 1 && n >= 1 && k >= 0 && splits && workspace_floats,
              "gemm_tn_workspace: bad arguments");
-  const int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128);
-  // About 1024 workgroups (4 per CU, one per SIMD each) in multiples of the
-  // XCD count, with at least 8 K-steps per workgroup.
-  int64_t s = (1024 + tiles - 1) / tiles;
+  const bool swap = gr_gemm::tn_swaps(m, n);
+  const int64_t pm = swap ? n : m, pn = swap ? m : n;
+  const auto t = gr_gemm::tn_tile(pm, pn, k);
+  const int64_t tiles = ((pm + t.bm - 1) / t.bm) * ((pn + t.bn - 1) / t.bn);
+  // Workgroups to fill the chip once (256 x 256 tiles, one a CU) or a few
+  // times, in multiples of the XCD count, with at least 64 rows each.
+  int64_t s = (t.target + tiles - 1) / tiles;
   s = (s + 7) / 8 * 8;
-  const int64_t max_s = std::max<int64_t>(1, k / (8 * 16));
+  const int64_t max_s = std::max<int64_t>(1, k / 64);
   if (s > max_s) s = max_s;
   if (s > 4096) s = 4096;
   if (s < 1) s = 1;
@@ -249,59 +122,46 @@ extern "C" int gr_gemm_tn(const float* a, int64_t lda, const float* b, int64_t l
              "gemm_tn: NULL pointer");
   hipStream_t s = gr::as_stream(stream);
   int64_t kchunk = (k + splits - 1) / splits;
-  kchunk = (kchunk + TK - 1) / TK * TK;
-  if (kchunk == 0) kchunk = TK;
+  kchunk = (kchunk + 15) / 16 * 16;
+  if (kchunk == 0) kchunk = 16;
   const int64_t used = k == 0 ? 1 : (k + kchunk - 1) / kchunk;
   GR_REQUIRE(used <= splits, "gemm_tn: internal chunking error");
   GR_REQUIRE(workspace_floats >= used * m * n,
              "gemm_tn: workspace of %lld floats, %lld needed", (long long)workspace_floats,
              (long long)(used * m * n));
-  // A narrow product (m <= 64 < n) runs as C^T = B^T A, so the narrow side
-  // falls on 64-column tiles instead of wasting rows of 128-row tiles; the
-  // partials are summed into C with a transposed store.
-  const bool swap = m <= 64 && n > 64;
+  const bool swap = tn_swaps(m, n);
   const float* pa = swap ? b : a;
   const float* pb = swap ? a : b;
   const int64_t pm = swap ? n : m, pn = swap ? m : n;
   const int64_t plda = swap ? ldb : lda, pldb = swap ? lda : ldb;
-  const bool va = (plda % 4 == 0) && (pm % 4 == 0) && (reinterpret_cast<uintptr_t>(pa) % 16 == 0);
-  const bool vb = (pldb % 4 == 0) && (pn % 4 == 0) && (reinterpret_cast<uintptr_t>(pb) % 16 == 0);
-  const bool narrow = pn <= 64;
-  // At most 32 columns (a 19- or 20-wide layer's dW): 32-column tiles, so the
-  // matrix cores do not work on 44 padded columns of 64; the product is then
-  // bound by streaming the wide operand.
-  const bool narrow32 = pn <= 32;
-  const int bn = narrow32 ? 32 : narrow ? 64 : TN;
-  const int tiles_m = (int)((pm + TM - 1) / TM);
-  const int tiles = tiles_m * (int)((pn + bn - 1) / bn);
+  const TnTile t = tn_tile(pm, pn, k);
+  const int tiles_m = (int)((pm + t.bm - 1) / t.bm);
+  const int64_t tiles = tiles_m * ((pn + t.bn - 1) / t.bn);
   const int64_t nwg = (used + kXcds - 1) / kXcds * kXcds * tiles;
   GR_REQUIRE(nwg <= INT32_MAX, "gemm_tn: too many workgroups");
   const dim3 grid((unsigned)nwg);
-#define GR_GT(VA_, VB_, BN_, BLK_)                                                             \
-  hipLaunchKernelGGL((gemm_tn_splitk<VA_, VB_, BN_, BLK_>), grid, dim3(256), 0, s, pa, plda, pb, \
-                     pldb, (int)pm, (int)pn, k, kchunk, (int)used, tiles_m, tiles, workspace)
-  // 32 x 32 blocks for 64-column tiles, and for 128-column tiles up to
-  // kTn32MaxK rows of K; 16 x 16 for 32-column tiles.
-  const bool b32 = k <= kTn32MaxK;
-  if (narrow32) {
-    if (va) GR_GT(4, 1, 32, 16); else GR_GT(1, 1, 32, 16);
-  } else if (narrow) {
-    if (va && vb) GR_GT(4, 4, 64, 32); else if (va) GR_GT(4, 1, 64, 32);
-    else if (vb) GR_GT(1, 4, 64, 32); else GR_GT(1, 1, 64, 32);
-  } else {
-    if (b32) {
-      if (va && vb) GR_GT(4, 4, 128, 32); else if (va) GR_GT(4, 1, 128, 32);
-      else if (vb) GR_GT(1, 4, 128, 32); else GR_GT(1, 1, 128, 32);
-    } else {
-      if (va && vb) GR_GT(4, 4, 128, 16); else if (va) GR_GT(4, 1, 128, 16);
-      else if (vb) GR_GT(1, 4, 128, 16); else GR_GT(1, 1, 128, 16);
-    }
-  }
+  const bool long_rows = plda >= (1 << 25) || pldb >= (1 << 25);
+#define GR_GT(WM, WN, MI, NJ)                                                                  \
+  do {                                                                                         \
+    if (long_rows)                                                                             \
+      hipLaunchKernelGGL((gr_bf3::gemm_tn_bf3<WM, WN, MI, NJ, true>), grid, dim3(WM * WN * 64), \
+                         0, s, pa, plda, pb, pldb, (int)pm, (int)pn, k, kchunk, (int)used,     \
+                         tiles_m, (int)tiles, workspace);                                      \
+    else                                                                                       \
+      hipLaunchKernelGGL((gr_bf3::gemm_tn_bf3<WM, WN, MI, NJ, false>), grid,                   \
+                         dim3(WM * WN * 64), 0, s, pa, plda, pb, pldb, (int)pm, (int)pn, k,    \
+                         kchunk, (int)used, tiles_m, (int)tiles, workspace);                   \
+  } while (0)
+  if (t.bm == 64) GR_GT(2, 2, 1, 1);
+  else if (t.bn == 32) GR_GT(4, 1, 1, 1);
+  else if (t.bn == 64) GR_GT(4, 1, 2, 2);
+  else if (t.bn == 128) GR_GT(2, 2, 2, 2);
+  else GR_GT(4, 2, 2, 4);
 #undef GR_GT
   GR_HIP_CHECK(hipGetLastError());
   const int64_t elems = m * n;
-  const unsigned blocks = (unsigned)std::min<int64_t>(4096, (elems + 255) / 256);
-  hipLaunchKernelGGL(sum_partials, dim3(blocks), dim3(256), 0, s, workspace, (int)used, pm, pn,
+  const unsigned blocks = (unsigned)std::min<int64_t>(16384, (elems + 63) / 64);
+  hipLaunchKernelGGL(sum_partials, dim3(blocks), dim3(kSumWaves * 64), 0, s, workspace, (int)used, pm, pn,
                      beta, (int)swap, c);
   GR_HIP_CHECK(hipGetLastError());
   return GR_OK;
@@ -1085,6 +945,95 @@ extern "C" int gr_gemm_nt(const float* a, int64_t lda, const float* b, int64_t l
   else
     err = dispatch_nt<1, 1>(a, lda, b, ldb, bias, c, ldc, m, (int)n, (int)k, s);
   GR_REQUIRE(err != hipErrorInvalidValue, "gemm_nt: too many workgroups for %lld rows",
+             (long long)m);
+  GR_HIP_CHECK(err);
+  return GR_OK;
+}
+
+// ---------------------------------------------------------------------------
+// The row-block product on split operands (gemm_nt_bf3): the input gradient
+// dx = dy W.  1.2 to 3 times as fast as gr_gemm_nt over the transform's shapes,
+// and closer to float64.  The forward product stays on gr_gemm_nt: its results
+// meet the ReLU and LeakyReLU kinks, and an output within rounding of one that
+// changed side would change the elementwise input gradients behind it by far
+// more than rounding; the gradients themselves meet none.
+namespace gr_gemm {
+
+template <int WM, int WN, int MI, int NJ>
+static hipError_t launch_split(const float* a, int64_t lda, const float* b, int64_t ldb,
+                            const float* bias, float* c, int64_t ldc, int64_t m, int n, int k,
+                            bool vec, hipStream_t s) {
+  constexpr int BM = WM * MI * 32, BN = WN * NJ * 32;
+  const int tiles_n = (n + BN - 1) / BN;
+  const int64_t grid = ((m + BM - 1) / BM + kXcds - 1) / kXcds * kXcds * tiles_n;
+  if (grid > INT32_MAX) return hipErrorInvalidValue;
+  const int store =
+      ldc >= (1 << 21) ? 0
+      : n % 4 == 0 && ldc % 4 == 0 && reinterpret_cast<uintptr_t>(c) % 16 == 0 ? 2 : 1;
+  const dim3 g((unsigned)grid), t(WM * WN * 64);
+  if (vec && k % 16 == 0)
+    hipLaunchKernelGGL((gr_bf3::gemm_nt_bf3<WM, WN, MI, NJ, 4, false>), g, t, 0, s, a, lda, b,
+                       ldb, bias, c, ldc, m, n, k, tiles_n, store);
+  else if (vec)
+    hipLaunchKernelGGL((gr_bf3::gemm_nt_bf3<WM, WN, MI, NJ, 4, true>), g, t, 0, s, a, lda, b,
+                       ldb, bias, c, ldc, m, n, k, tiles_n, store);
+  else
+    hipLaunchKernelGGL((gr_bf3::gemm_nt_bf3<WM, WN, MI, NJ, 1, true>), g, t, 0, s, a, lda, b,
+                       ldb, bias, c, ldc, m, n, k, tiles_n, store);
+  return hipGetLastError();
+}
+
+// Tile by the product's shape, as measured (us; m x n x k):
+//   n <= 32: 128 x 32 (100k x 20 x 256 22; 128 x 64 30);
+//   n <= 64: 128 x 64 (200k x 48 x 256 51, 50k x 64 x 256 18.6);
+//   else 128 x 128 (200k x 256 x 48 49, 100k x 256 x 256 84);
+//   128 x 256 for n > 128 and k >= 128 once there are four rounds of them
+//     (two a CU: 1M x 256 x 256 765 against 850 for 128 x 128 and 925 for
+//     256 x 256);
+//   256 x 256 for k >= 512, where a tile's start and end weigh less than the
+//     operands it re-reads (250k x 256 x 1024 643, 128 x 256 655);
+//   64 x 64, or 64 x 32, where those leave CUs without a tile (10k x 64 x 128
+//     7.9, 5k x 128 x 300 11; 128 x 128 10 and 21).
+static hipError_t dispatch_split(const float* a, int64_t lda, const float* b, int64_t ldb,
+                              const float* bias, float* c, int64_t ldc, int64_t m, int n, int k,
+                              bool vec, hipStream_t s) {
+#define GR_NT(...) return launch_split<__VA_ARGS__>(a, lda, b, ldb, bias, c, ldc, m, n, k, vec, s)
+  const int64_t m128 = (m + 127) / 128, m256 = (m + 255) / 256;
+  const int64_t n128 = (n + 127) / 128, n256 = (n + 255) / 256;
+  if (n <= 32) {
+    if (m128 < 256) GR_NT(2, 1, 1, 1);
+    GR_NT(2, 1, 2, 1);
+  }
+  if (n <= 64) {
+    if (m128 < 256) GR_NT(2, 2, 1, 1);
+    GR_NT(4, 1, 1, 2);
+  }
+  if (m128 * n128 < 256) GR_NT(2, 2, 1, 1);
+  if (n > 128 && k >= 512 && m256 * n256 >= 512) GR_NT(4, 2, 2, 4);
+  if (n > 128 && k >= 128 && m128 * n256 >= 2048) GR_NT(2, 2, 2, 4);
+  GR_NT(2, 2, 2, 2);
+#undef GR_NT
+}
+
+}  // namespace gr_gemm
+
+extern "C" int gr_gemm_nt_split(const float* a, int64_t lda, const float* b, int64_t ldb,
+                                int64_t m, int64_t n, int64_t k, const float* bias, float* c,
+                                int64_t ldc, void* stream) {
+  using namespace gr_gemm;
+  gr::clear_error();
+  GR_REQUIRE(m >= 0 && n >= 1 && k >= 1 && n <= (1 << 20) && k <= (1 << 24),
+             "gemm_nt_split: bad shape %lld x %lld x %lld", (long long)m, (long long)n,
+             (long long)k);
+  GR_REQUIRE(lda >= k && ldb >= k && ldc >= n, "gemm_nt_split: leading dimension too small");
+  if (m == 0) return GR_OK;
+  GR_REQUIRE(a != nullptr && b != nullptr && c != nullptr, "gemm_nt_split: NULL pointer");
+  const bool vec = k % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 &&
+                   reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(b) % 16 == 0;
+  const hipError_t err = dispatch_split(a, lda, b, ldb, bias, c, ldc, m, (int)n, (int)k, vec,
+                                        gr::as_stream(stream));
+  GR_REQUIRE(err != hipErrorInvalidValue, "gemm_nt_split: too many workgroups for %lld rows",
              (long long)m);
   GR_HIP_CHECK(err);
   return GR_OK;

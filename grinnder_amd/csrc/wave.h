@@ -173,7 +173,9 @@ __device__ __forceinline__ void quad_transpose(float& v0, float& v1, float& v2, 
 // family's raw-buffer format (the value composable_kernel's ck.hpp uses).
 constexpr uint32_t kBufferDrop = 0x80000000u;  // past any resource made below
 
-// `bytes` < 2^31; the base must be wave-uniform.
+// `bytes` < 2^31; the base must be wave-uniform.  The whole offset of an access
+// goes through the lane's register: the hardware's range check covers that, not
+// surely the scalar offset.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
                                            0x00020000);

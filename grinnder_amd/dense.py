@@ -2,11 +2,12 @@
 
 PyG's GCNConv / GATConv (grinnder/nn/gcn.py:53-56, grinnder/nn/gat.py:54-61)
 apply a bias-free ``Linear`` to the node features.  All three of its
-products run on this library's fp32 MFMA kernels: the forward x Wᵀ (+ b) and
-the input gradient dy W on ``gr_gemm_nt`` (row-block tiles, K-contiguous
-operands), the weight gradient dW = dyᵀ x, which reduces over all K node rows
-of the partition with M, N <= a few hundred, on ``gr_gemm_tn`` (split-K,
-partials summed in a fixed order).
+products run on this library's MFMA kernels: the forward x Wᵀ (+ b) on
+``gr_gemm_nt`` (row-block tiles, K-contiguous operands, fp32 instructions), the
+input gradient dy W on ``gr_gemm_nt_split`` and the weight gradient dW = dyᵀ x,
+which reduces over all K node rows of the partition with M, N <= a few hundred,
+on ``gr_gemm_tn`` (split-K, partials summed in a fixed order), both on operands
+split into bf16 pieces.
 
 ``bias_ln_act`` is the dense counterpart of the fused aggregation epilogue:
 LayerNorm + ReLU after a GCN layer that aggregates first and multiplies
@@ -98,8 +99,17 @@ def gemm_tn(a: Tensor, b: Tensor, out: Optional[Tensor] = None, beta: float = 0.
     return out
 
 
+def gemm_nt_split(a: Tensor, b: Tensor, bias: Optional[Tensor] = None,
+                  out: Optional[Tensor] = None) -> Tensor:
+    """gemm_nt on operands split into three bf16 pieces each (24 bits, fp32
+    sums; results no further from float64): faster, with other rounding.  The
+    backward's products run on it; the forward's keep gemm_nt's rounding, so
+    outputs next to an activation's kink keep their side."""
+    return gemm_nt(a, b, bias, out, _entry="gr_gemm_nt_split")
+
+
 def gemm_nt(a: Tensor, b: Tensor, bias: Optional[Tensor] = None,
-            out: Optional[Tensor] = None) -> Tensor:
+            out: Optional[Tensor] = None, _entry: str = "gr_gemm_nt") -> Tensor:
     """C = a bᵀ (+ bias) for a [M, K] and b [N, K] fp32 device matrices with
     unit column stride (rows may be strided) on the matrix cores, or, for a
     short reduction (K <= 64, N >= 64), as a stream of C's rows on the vector
@@ -131,15 +141,15 @@ def gemm_nt(a: Tensor, b: Tensor, bias: Optional[Tensor] = None,
         return out
     if k == 0:
         return out.copy_(bias.expand(m, n) if bias is not None else torch.zeros_like(out))
-    _lib.call("gr_gemm_nt", a.data_ptr(), max(a.stride(0), k), b.data_ptr(),
+    _lib.call(_entry, a.data_ptr(), max(a.stride(0), k), b.data_ptr(),
               max(b.stride(0), k), m, n, k, _lib.ptr(bias), out.data_ptr(),
               max(out.stride(0), n), _lib.stream_handle())
     return out
 
 
 class _Linear(torch.autograd.Function):
-    """y = x W^T (+ b) and dx = dy W (gr_gemm_nt), dW = dy^T x (gr_gemm_tn),
-    db = sum dy.
+    """y = x W^T (+ b) (gr_gemm_nt), dx = dy W (gr_gemm_nt_split), dW = dy^T x
+    (gr_gemm_tn), db = sum dy.
     `reuse` (a one-element list, or None) holds y as an earlier forward
     computed it from the same x, W and b: it is returned instead of being
     recomputed, and the backward is the same."""
@@ -171,7 +181,7 @@ class _Linear(torch.autograd.Function):
         rows, dout, din = gy2.size(0), weight.size(0), weight.size(1)
         if ctx.needs_input_grad[0]:
             with dense_region("dx", rows, dout, din):
-                dx = gemm_nt(gy2, weight.t().contiguous()).reshape(ctx.in_shape)
+                dx = gemm_nt_split(gy2, weight.t().contiguous()).reshape(ctx.in_shape)
         if ctx.needs_input_grad[1]:
             with dense_region("dw", rows, dout, din):
                 dw = gemm_tn(gy2, x2)
@@ -183,8 +193,8 @@ class _Linear(torch.autograd.Function):
 
 def linear(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None,
            reuse: Optional[Tensor] = None) -> Tensor:
-    """``F.linear`` on the library's MFMA kernels (GPU): forward and input
-    gradient on gr_gemm_nt, weight gradient on the split-K gr_gemm_tn.
+    """``F.linear`` on the library's MFMA kernels (GPU): forward on gr_gemm_nt,
+    input gradient on gr_gemm_nt_split, weight gradient on the split-K gr_gemm_tn.
     `reuse`: this product as an earlier forward formed it from the same
     operands (rows [-1, out]); it is returned instead of recomputed, with the
     same backward."""
@@ -237,7 +247,7 @@ class _BiasLNAct(torch.autograd.Function):
                 shift=ctx.bias, rowdot=rowdot)
         else:
             if prod is not None:
-                gout = gout + gemm_nt(prod[0], prod[1].t().contiguous())
+                gout = gout + gemm_nt_split(prod[0], prod[1].t().contiguous())
             gh, dgamma, dbeta, db = ln_act_backward(gout, h, mean, rstd, g, bt, ctx.has_bias,
                                                     ctx.act, shift=ctx.bias, rowdot=rowdot)
         if ctx.sink is not None:
@@ -314,7 +324,7 @@ class _LinearLNAct(torch.autograd.Function):
         rows, din, dout = x.size(0), x.size(1), w.size(0)
         if ctx.needs_input_grad[0]:
             with dense_region("dx", rows, dout, din):
-                dx = gemm_nt(gh, w.t().contiguous())
+                dx = gemm_nt_split(gh, w.t().contiguous())
         if ctx.needs_input_grad[1]:
             with dense_region("dw", rows, dout, din):
                 dw = gemm_tn(gh, x)

@@ -395,8 +395,10 @@ int gr_xent_forward(const float* logits, int64_t ld, int64_t rows,
 /* ------------------------------------------------------------------------ */
 
 /* C[M, N] = A^T B (+ beta * C) with A [K, M] (lda-strided rows) and B [K, N]
- * (ldb-strided rows), fp32 on the matrix cores, split over K into `splits`
- * chunks whose partial tiles are summed in chunk order (deterministic).  This
+ * (ldb-strided rows), on the matrix cores with every operand split into three
+ * bf16 pieces (24 bits, fp32 sums; no further from float64 than fp32 products,
+ * infinities and NaN as in fp32), over `splits` chunks of K whose partial
+ * tiles are summed in a fixed order (deterministic).  This
  * is the weight gradient dW = dZ^T X of the conv's dense transform (the
  * Linear inside PyG GCNConv / GATConv of grinnder/nn/gcn.py:53-56 and
  * grinnder/nn/gat.py:54-61), whose K is the partition's row count.
@@ -419,6 +421,12 @@ int gr_gemm_tn(const float* a, int64_t lda, const float* b, int64_t ldb,
 int gr_gemm_nt(const float* a, int64_t lda, const float* b, int64_t ldb,
                int64_t m, int64_t n, int64_t k, const float* bias, float* c,
                int64_t ldc, void* stream);
+
+/* gr_gemm_nt on split operands (as gr_gemm_tn): the input gradient dx = dy W
+ * (B = W^T) of the same Linear. */
+int gr_gemm_nt_split(const float* a, int64_t lda, const float* b, int64_t ldb,
+                     int64_t m, int64_t n, int64_t k, const float* bias,
+                     float* c, int64_t ldc, void* stream);
 
 /* Dense layer transform with the LayerNorm epilogue in the GEMM accumulators:
  *   h = x W^T + bias, out = act(LayerNorm(h; gamma, beta, eps)), mean, rstd
