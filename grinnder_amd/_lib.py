@@ -93,6 +93,11 @@ _SIGNATURES = {
                                _i64, _P],
     "gr_gat_backward_dst": [_P, _i64, _P, _i64, _P, _P, _P, _P, _i64, _i64, _P, _P, _P, _i64,
                             _P],
+    "gr_gat_heads_workspace": [_i64, _i64, _i32, _P],
+    "gr_gat_heads_forward": [_P, _i64, _P, _i64, _P, _P, _i64, _P, _P, _i64, _i64, _P, _P, _P,
+                             _P, _P, _P, _i64, _i64, _P],
+    "gr_gat_heads_backward": [_P, _i64, _P, _i64, _P, _P, _i64, _P, _P, _P, _P, _P, _i64, _i64,
+                              _i64, _P, _P, _P, _P, _P, _P, _P, _i64, _i64, _P],
     "gr_io_create": [_i32, _P],
     "gr_io_destroy": [_P],
     "gr_io_submit": [_P, _i32, ctypes.c_char_p, _P, _i64, _i64, _P],

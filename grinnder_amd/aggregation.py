@@ -592,6 +592,19 @@ def _gat_records_ok(hs: Tensor, heads: int, channels: int) -> bool:
     return channels <= 256
 
 
+def _gat_heads_ok(hs: Tensor, heads: int, channels: int) -> bool:
+    """Several heads whose lanes gr_gat_heads_forward / _backward hold: H times
+    the power of two at or above a head's vectors, at most 512 lanes (256 a
+    head); wider rows take the general kernels."""
+    if not 2 <= heads <= 16:
+        return False
+    rows = hs.data_ptr() | 4 * hs.stride(0)
+    vec = (4 if channels % 4 == 0 and rows % 16 == 0
+           else 2 if channels % 2 == 0 and rows % 8 == 0 else 1)
+    lanes = 1 << ((channels + vec - 1) // vec - 1).bit_length()
+    return lanes <= 256 and heads * lanes <= 512 and heads * channels <= 1024
+
+
 def _attention_backward(plan: DevicePlan, hs: Tensor, a_src: Tensor, a_dst: Tensor, s: Tensor,
                         d: Tensor, alpha_or_m: Tensor, den: Tensor, go: Tensor, cdot: Tensor,
                         H: int, C: int, records: bool, zsink: Optional[ProjectedSink]):
@@ -695,7 +708,9 @@ class _GATAttention(torch.autograd.Function):
                 plan: DevicePlan, heads: int, channels: int, concat: bool,
                 s_pre: Optional[Tensor] = None, d_pre: Optional[Tensor] = None,
                 sink: Optional[RowDotSink] = None, zsink: Optional[ProjectedSink] = None,
-                token: Optional[Tensor] = None, zx_pre: Optional[Tensor] = None) -> Tensor:
+                token: Optional[Tensor] = None, zx_pre: Optional[Tensor] = None,
+                keep: bool = True) -> Tensor:
+        # keep: a backward may follow (several heads keep its state then).
         # zsink: hs is the matrix of all partitions' rows ([N, H*C], s_pre
         # [N, H] alike), read in place through zsink.gidx; the backward adds
         # dHs into zsink.dz at zsink.rows.  zx_pre: hs's packed lines
@@ -724,6 +739,9 @@ class _GATAttention(torch.autograd.Function):
             d = torch.empty((B, H), dtype=torch.float32, device=dev)
             _lib.call("gr_gat_scores", hs.data_ptr(), hs.stride(0), E, B, H, C, a_src.data_ptr(),
                       a_dst.data_ptr(), s.data_ptr(), d.data_ptr(), stream)
+        if zsink is None and _gat_heads_ok(hs, H, C):
+            return _GATAttention._forward_heads(ctx, hs, a_src, a_dst, bias, plan, H, C, concat,
+                                                s, d, region, att_src.shape, keep)
         m = torch.empty((B, H), dtype=torch.float32, device=dev)
         den = torch.empty((B, H), dtype=torch.float32, device=dev)
         # One head: alpha is not stored; the backward recomputes it from the
@@ -805,6 +823,77 @@ class _GATAttention(torch.autograd.Function):
         return out
 
     @staticmethod
+    def _forward_heads(ctx, hs, a_src, a_dst, bias, plan, H, C, concat, s, d, region, att_shape,
+                       keep):
+        """Several heads in one pass over the edges (gr_gat_heads_forward); with
+        `keep` it also leaves the state its backward needs."""
+        dev = hs.device
+        HC, B = H * C, plan.num_dst
+        f = plan.fwd
+        width = ctypes.c_int64(0)
+        _lib.call("gr_gat_heads_workspace", H, C, int(keep), ctypes.addressof(width))
+        ws = _workspace(f.n_slots, width.value, dev)
+        fused_bias = concat and bias is not None
+        y = torch.empty((B, HC), dtype=torch.float32, device=dev) if fused_bias else None
+        o = torch.empty((B, HC), dtype=torch.float32, device=dev) if keep or y is None else None
+        state = torch.empty((B, H, 4), dtype=torch.float32, device=dev) if keep else None
+        nrow = torch.empty((B, HC), dtype=torch.float32, device=dev) if keep else None
+        b = bias.contiguous() if fused_bias else None
+        _lib.call("gr_gat_heads_forward", f.units.data_ptr(), f.n_units,
+                  f.fixups.data_ptr() if f.n_fix else None, f.n_fix, plan.idx.data_ptr(),
+                  hs.data_ptr(), hs.stride(0), s.data_ptr(), d.data_ptr(), H, C, _lib.ptr(b),
+                  _lib.ptr(state), _lib.ptr(nrow), _lib.ptr(o), _lib.ptr(y), _lib.ptr(ws),
+                  0 if ws is None else ws.numel(), f.n_slots, _lib.stream_handle())
+        region.__exit__(None, None, None)
+        if concat:
+            y = o if y is None else y
+        else:
+            y = o.view(B, H, C).mean(dim=1)
+            if bias is not None:
+                y = y + bias
+        if keep:
+            ctx.save_for_backward(hs, a_src, a_dst, s, o, nrow, state)
+        ctx.several = True
+        ctx.plan = plan
+        ctx.shape = (H, C, concat)
+        ctx.has_bias = bias is not None
+        ctx.att_shape = att_shape
+        return y
+
+    @staticmethod
+    def _backward_heads(ctx, gy: Tensor):
+        hs, a_src, a_dst, s, o, nrow, state = ctx.saved_tensors
+        plan: DevicePlan = ctx.plan
+        H, C, concat = ctx.shape
+        HC = H * C
+        E, B = plan.num_src, plan.num_dst
+        dev = hs.device
+        gy = gy.contiguous()
+        go = gy if concat else (gy / H).unsqueeze(1).expand(B, H, C).reshape(B, HC).contiguous()
+        db = column_sum(gy) if ctx.has_bias else None
+        nnz = plan.nnz
+        bw = plan.bwd
+        with KernelTimer.region(
+                "gat_bwd", nnz * (8 * HC + 16 * H + 8) + E * (4 * HC + 4 * H)
+                + B * (4 * HC + 4 * H), nnz, HC):
+            rec = torch.empty((B, H, 4), dtype=torch.float32, device=dev)
+            dhs = torch.empty((E, HC), dtype=torch.float32, device=dev)
+            ds = torch.empty((E, H), dtype=torch.float32, device=dev)
+            dd = torch.empty((B, H), dtype=torch.float32, device=dev)
+            ws = _workspace(bw.n_slots, (HC + 3) // 4 * 4 + (H + 3) // 4 * 4, dev)
+            _lib.call("gr_gat_heads_backward", bw.units.data_ptr(), bw.n_units,
+                      bw.fixups.data_ptr() if bw.n_fix else None, bw.n_fix,
+                      plan.row_idx.data_ptr(), hs.data_ptr(), hs.stride(0), s.data_ptr(),
+                      go.data_ptr(), o.data_ptr(), nrow.data_ptr(), state.data_ptr(), B, H, C,
+                      a_src.data_ptr(), a_dst.data_ptr(), rec.data_ptr(), dd.data_ptr(),
+                      dhs.data_ptr(), ds.data_ptr(), _lib.ptr(ws),
+                      0 if ws is None else ws.numel(), bw.n_slots, _lib.stream_handle())
+        datt_src = column_sum(hs, ds, C)
+        datt_dst = column_sum(hs[:B], dd, C)
+        return (dhs, datt_src.view(ctx.att_shape), datt_dst.view(ctx.att_shape), db,
+                None, None, None, None, None, None, None, None, None, None, None)
+
+    @staticmethod
     def _backward_narrow(ctx, gy: Tensor):
         hs, a_src, a_dst, zx, fstate, out, dvec, b = ctx.saved_tensors
         plan: DevicePlan = ctx.plan
@@ -837,12 +926,14 @@ class _GATAttention(torch.autograd.Function):
         datt_src = column_sum(hs, ds, C)
         datt_dst = column_sum(hs[:B], dd, C)
         return (dhs, datt_src.view(ctx.att_shape), datt_dst.view(ctx.att_shape), db,
-                None, None, None, None, None, None, None, None, None, None)
+                None, None, None, None, None, None, None, None, None, None, None)
 
     @staticmethod
     def backward(ctx, gy: Tensor):
         if getattr(ctx, "narrow", False):
             return _GATAttention._backward_narrow(ctx, gy)
+        if getattr(ctx, "several", False):
+            return _GATAttention._backward_heads(ctx, gy)
         hs, a_src, a_dst, s, d, alpha_or_m, den, o = ctx.saved_tensors
         plan: DevicePlan = ctx.plan
         H, C, concat = ctx.shape
@@ -870,7 +961,7 @@ class _GATAttention(torch.autograd.Function):
         dhs, datt_src, datt_dst = _attention_backward(plan, hs, a_src, a_dst, s, d, alpha_or_m,
                                                       den, go, cdot, H, C, ctx.records, zsink)
         return (dhs, datt_src.view(ctx.att_shape), datt_dst.view(ctx.att_shape), db,
-                None, None, None, None, None, None, None, None, None, None)
+                None, None, None, None, None, None, None, None, None, None, None)
 
 
 def gat_scores(hs: Tensor, att_src: Tensor, att_dst: Tensor, heads: int, channels: int,
@@ -940,9 +1031,11 @@ def gat_attention(hs: Tensor, adj: Adjacency, att_src: Tensor, att_dst: Tensor,
                                    s, d, rowdot_sink, sink, sink.token)
     if hs.size(0) != plan.num_src:
         raise ValueError(f"hs has {hs.size(0)} rows, adjacency has {plan.num_src} columns")
+    keep = torch.is_grad_enabled() and any(
+        t is not None and t.requires_grad for t in (hs, att_src, att_dst, bias))
     if scores is None:
         return _GATAttention.apply(hs, att_src, att_dst, bias, plan, heads, channels, concat,
-                                   None, None, rowdot_sink)
+                                   None, None, rowdot_sink, None, None, None, keep)
     s, d = scores[0], scores[1]
     if tuple(s.shape) != (plan.num_src, heads) or tuple(d.shape) != (plan.num_dst, heads):
         raise ValueError("gat_attention: scores do not match the adjacency and heads")
@@ -950,7 +1043,7 @@ def gat_attention(hs: Tensor, adj: Adjacency, att_src: Tensor, att_dst: Tensor,
     if zx is not None and tuple(zx.shape) != (plan.num_src, 32):
         raise ValueError("gat_attention: packed rows do not match the adjacency")
     return _GATAttention.apply(hs, att_src, att_dst, bias, plan, heads, channels, concat, s, d,
-                               rowdot_sink, None, None, zx)
+                               rowdot_sink, None, None, zx, keep)
 
 
 class _GATAttentionLN(torch.autograd.Function):

@@ -30,6 +30,7 @@ SOURCES = [
     "aggregate.hip",
     "gat.hip",
     "gat_narrow.hip",
+    "gat_heads.hip",
     "gemm.hip",
     "loss.hip",
 ]

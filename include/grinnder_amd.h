@@ -677,6 +677,36 @@ int gr_gat_backward_dst(const int32_t* units, int64_t n_units,
                         float* dd, float* dhs, float* workspace,
                         int64_t n_slots, void* stream);
 
+/* Several heads, one pass over the edges each way (the attention, edge softmax
+ * and aggregation of PyG GATConv, grinnder/nn/gat.py:54-61,73, and their
+ * backward).  units / fixups / idx / row_idx as gr_gat_forward and
+ * gr_gat_backward_src; 2 to 16 heads H of C channels, H * C <= 1024, whose
+ * lanes (H times the power of two at or above C / 4, or C / 2, or C for rows
+ * that 16- or 8-byte accesses do not take) are at most 512, a head's at most 256.
+ * Forward: o = O and / or y = O + bias (either may be NULL, not both).  With
+ * state ([rows, H] float4) and nrow ([rows, H*C]) it also keeps what the
+ * backward needs: (d, m, den, S) and N = sum of alpha Hs over the edges with
+ * s + d <= 0, S the same sum of alpha.
+ * Backward, from go = dL/dO and the forward's o, nrow and state: rec ([n_dst,
+ * H] float4, scratch), dd [n_dst, H] and ds (the gradients of d and s), and dhs
+ * [rows of the plan, H*C] with both attention vectors' parts in it.
+ * Workspace: n_slots times gr_gat_heads_workspace's floats (with_state != 0
+ * for a forward that keeps state; the backward needs no more than that). */
+int gr_gat_heads_workspace(int64_t H, int64_t C, int32_t with_state,
+                           int64_t* floats_per_slot);
+int gr_gat_heads_forward(const int32_t* units, int64_t n_units, const int32_t* fixups,
+                         int64_t n_fix, const int32_t* idx, const float* hs, int64_t ldh,
+                         const float* s, const float* d, int64_t H, int64_t C,
+                         const float* bias, float* state, float* nrow, float* o, float* y,
+                         float* ws, int64_t ws_floats, int64_t n_slots, void* stream);
+int gr_gat_heads_backward(const int32_t* units, int64_t n_units, const int32_t* fixups,
+                          int64_t n_fix, const int32_t* row_idx, const float* hs, int64_t ldh,
+                          const float* s, const float* go, const float* o, const float* nrow,
+                          const float* state, int64_t n_dst, int64_t H, int64_t C,
+                          const float* att_src, const float* att_dst, float* rec, float* dd,
+                          float* dhs, float* ds, float* ws, int64_t ws_floats,
+                          int64_t n_slots, void* stream);
+
 /* ------------------------------------------------------------------------ */
 /* Host <-> storage I/O (grinnder._C.IoUringEngine)                          */
 /* ------------------------------------------------------------------------ */

@@ -1,0 +1,85 @@
+"""Several attention heads in one pass (csrc/gat_heads.hip) against the oracle:
+every lane layout (heads and channels around powers of two, 16-, 8- and 4-byte
+rows, one to eight chunks a row, edge slots), split and empty rows, and the
+forward without a backward."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import oracle
+from grinnder_amd.aggregation import _gat_heads_ok, gat_attention
+from grinnder_amd.data.adjacency import Adjacency
+from tests.graphs import TOL, max_abs_norm_err, random_bipartite
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # (heads, channels, one-pass kernels)
+    (2, 1, True), (16, 1, True), (2, 2, True), (3, 5, True), (5, 16, True), (7, 12, True),
+    (8, 8, True), (8, 23, True), (8, 32, True), (2, 116, True), (2, 69, True), (4, 49, True),
+    (2, 256, True), (2, 512, True), (2, 129, True), (4, 130, True), (16, 64, True),
+    (15, 68, True), (6, 6, True), (3, 257, False), (2, 511, False),
+]
+
+
+def _inputs(H, C, concat, rows=260, sources=400, seg_len=64):
+    rowptr, col, val = random_bipartite(rows, sources, 9, seed=H * 7 + C, long_rows=2,
+                                        long_len=300)
+    adj = Adjacency(rowptr, col, val, (rows, sources), seg_len=seg_len)
+    g = torch.Generator().manual_seed(H * 100 + C)
+    hs = torch.randn(sources, H * C, generator=g)
+    att_src = torch.randn(1, H, C, generator=g) * C ** -0.5
+    att_dst = torch.randn(1, H, C, generator=g) * C ** -0.5
+    width = H * C if concat else C
+    return rowptr, col, adj, hs, att_src, att_dst, torch.randn(width, generator=g), \
+        torch.randn(rows, width, generator=g)
+
+
+@pytest.mark.parametrize("H,C,one_pass", CASES)
+@pytest.mark.parametrize("concat,offset", [(True, 0), (True, 1), (True, 2), (False, 0)])
+def test_heads_match_oracle(gpu, H, C, one_pass, concat, offset):
+    """offset: hs starts that many floats past 16-byte alignment."""
+    rowptr, col, adj, hs, a_s, a_d, bias, gy = _inputs(H, C, concat)
+    buf = torch.empty(hs.numel() + offset, device=gpu)
+    hs_d = buf[offset:].view(hs.shape)
+    hs_d.copy_(hs)
+    if offset == 0:
+        assert _gat_heads_ok(hs_d, H, C) == one_pass
+    hs_d = hs_d.detach().requires_grad_(True)
+    as_d, ad_d, b_d = (t.to(gpu).requires_grad_(True) for t in (a_s, a_d, bias))
+    y = gat_attention(hs_d, adj, as_d, ad_d, b_d, H, C, concat)
+    y.backward(gy.to(gpu))
+    ref, alpha, tpre = oracle.gat_forward(rowptr, col, hs, H, C, a_s, a_d, bias, concat)
+    dhs, das, dad, db = oracle.gat_backward(rowptr, col, hs, H, C, a_s, a_d, concat, alpha, tpre,
+                                            gy)
+    assert max_abs_norm_err(y, ref) <= TOL
+    assert max_abs_norm_err(hs_d.grad, dhs) <= TOL
+    assert max_abs_norm_err(as_d.grad.reshape(-1), torch.as_tensor(das).reshape(-1)) <= TOL
+    assert max_abs_norm_err(ad_d.grad.reshape(-1), torch.as_tensor(dad).reshape(-1)) <= TOL
+    assert max_abs_norm_err(b_d.grad, db) <= TOL
+    with torch.no_grad():
+        again = gat_attention(hs_d, adj, as_d, ad_d, b_d, H, C, concat)
+    assert torch.equal(again, y.detach())
+
+
+@pytest.mark.parametrize("H,C", [(8, 8), (2, 64), (4, 130)])
+def test_heads_extreme_logits(gpu, H, C):
+    """Logits of several hundred keep the softmax finite (the running maximum
+    is taken off before the exponential), rows without edges give the bias,
+    and a NaN source reaches only the rows that read it."""
+    rowptr, col, adj, hs, a_s, a_d, bias, _ = _inputs(H, C, True)
+    out = gat_attention((hs * 200).to(gpu), adj, a_s.to(gpu), a_d.to(gpu), bias.to(gpu), H, C)
+    ref = oracle.gat_forward(rowptr, col, hs * 200, H, C, a_s, a_d, bias, True)[0]
+    assert max_abs_norm_err(out, ref) <= 1e-4  # a logit of 1e3 has 6e-5 of rounding in it
+    empty = rowptr[1:] == rowptr[:-1]
+    assert bool(empty.any())
+    assert torch.equal(out.cpu()[empty], bias.expand(int(empty.sum()), -1))
+    bad = hs.clone()
+    bad[399] = float("nan")
+    reads = torch.zeros(260, dtype=torch.bool)
+    rows = torch.repeat_interleave(torch.arange(260), rowptr[1:] - rowptr[:-1])
+    reads[rows[col == 399]] = True
+    got = gat_attention(bad.to(gpu), adj, a_s.to(gpu), a_d.to(gpu), bias.to(gpu), H, C).cpu()
+    assert bool(got[~reads].isfinite().all()) and bool(got[reads].isnan().all())
