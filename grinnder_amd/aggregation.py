@@ -593,12 +593,23 @@ def _gat_records_ok(hs: Tensor, heads: int, channels: int) -> bool:
 
 
 def _gat_heads_ok(hs: Tensor, heads: int, channels: int) -> bool:
-    """Several heads whose lanes gr_gat_heads_forward / _backward hold: H times
-    the power of two at or above a head's vectors, at most 512 lanes (256 a
-    head); wider rows take the general kernels."""
+    """Whether the attention runs in one online-softmax pass each way
+    (gr_gat_heads_forward / _backward).
+
+    Several heads: where their lanes fit, heads times the power of two at or
+    above a head's vectors, at most 512 lanes (256 a head); wider rows take the
+    general kernels.  One head: 36..128 channels on 16-byte rows, where the
+    one-head kernels run rows of up to 32 edges and longer ones as two launches
+    (us forward and backward / forward alone, theirs first: 48 channels over 2M
+    edges, 100k rows 327/133 and 255/102, 128 channels 447/170 and 400/155).
+    Up to 32 channels half the lanes would idle (28: 306/79 and 261/107, 176/48
+    and 246/50 for 1M edges, 30k rows), and past 128 a wavefront has one edge
+    slot either way (164: 306/121 and 338/134 there)."""
+    rows = hs.data_ptr() | 4 * hs.stride(0)
+    if heads == 1:
+        return channels % 4 == 0 and 32 < channels <= 64 and rows % 16 == 0
     if not 2 <= heads <= 16:
         return False
-    rows = hs.data_ptr() | 4 * hs.stride(0)
     vec = (4 if channels % 4 == 0 and rows % 16 == 0
            else 2 if channels % 2 == 0 and rows % 8 == 0 else 1)
     lanes = 1 << ((channels + vec - 1) // vec - 1).bit_length()
@@ -741,7 +752,8 @@ class _GATAttention(torch.autograd.Function):
                       a_dst.data_ptr(), s.data_ptr(), d.data_ptr(), stream)
         if zsink is None and _gat_heads_ok(hs, H, C):
             return _GATAttention._forward_heads(ctx, hs, a_src, a_dst, bias, plan, H, C, concat,
-                                                s, d, region, att_src.shape, keep)
+                                                s, d, region, att_src.shape, keep,
+                                                sink)
         m = torch.empty((B, H), dtype=torch.float32, device=dev)
         den = torch.empty((B, H), dtype=torch.float32, device=dev)
         # One head: alpha is not stored; the backward recomputes it from the
@@ -824,15 +836,16 @@ class _GATAttention(torch.autograd.Function):
 
     @staticmethod
     def _forward_heads(ctx, hs, a_src, a_dst, bias, plan, H, C, concat, s, d, region, att_shape,
-                       keep):
-        """Several heads in one pass over the edges (gr_gat_heads_forward); with
-        `keep` it also leaves the state its backward needs."""
+                       keep, sink):
+        """One pass over the edges (gr_gat_heads_forward); with `keep` it also
+        leaves the state its backward needs."""
         dev = hs.device
         HC, B = H * C, plan.num_dst
         f = plan.fwd
         width = ctypes.c_int64(0)
         _lib.call("gr_gat_heads_workspace", H, C, int(keep), ctypes.addressof(width))
         ws = _workspace(f.n_slots, width.value, dev)
+        concat = concat or H == 1
         fused_bias = concat and bias is not None
         y = torch.empty((B, HC), dtype=torch.float32, device=dev) if fused_bias else None
         o = torch.empty((B, HC), dtype=torch.float32, device=dev) if keep or y is None else None
@@ -853,8 +866,9 @@ class _GATAttention(torch.autograd.Function):
                 y = y + bias
         if keep:
             ctx.save_for_backward(hs, a_src, a_dst, s, o, nrow, state)
-        ctx.several = True
+        ctx.one_pass = True
         ctx.plan = plan
+        ctx.sink = sink
         ctx.shape = (H, C, concat)
         ctx.has_bias = bias is not None
         ctx.att_shape = att_shape
@@ -871,6 +885,8 @@ class _GATAttention(torch.autograd.Function):
         gy = gy.contiguous()
         go = gy if concat else (gy / H).unsqueeze(1).expand(B, H, C).reshape(B, HC).contiguous()
         db = column_sum(gy) if ctx.has_bias else None
+        if ctx.sink is not None:
+            ctx.sink.cdot = None  # the row pass has O at hand and forms c itself
         nnz = plan.nnz
         bw = plan.bwd
         with KernelTimer.region(
@@ -932,7 +948,7 @@ class _GATAttention(torch.autograd.Function):
     def backward(ctx, gy: Tensor):
         if getattr(ctx, "narrow", False):
             return _GATAttention._backward_narrow(ctx, gy)
-        if getattr(ctx, "several", False):
+        if getattr(ctx, "one_pass", False):
             return _GATAttention._backward_heads(ctx, gy)
         hs, a_src, a_dst, s, d, alpha_or_m, den, o = ctx.saved_tensors
         plan: DevicePlan = ctx.plan

@@ -1,5 +1,6 @@
-// GAT attention with several heads for gfx950: one pass over the edges each
-// way (semantics as gat.hip: PyG GATConv, grinnder/nn/gat.py:54-61,69-78).
+// GAT attention with several heads, or one of 36 to 64 channels, for gfx950:
+// one pass over the edges each way (semantics as gat.hip: PyG GATConv,
+// grinnder/nn/gat.py:54-61,69-78).
 //
 // Lanes are laid out by head: head h owns LPH consecutive lane positions (LPH
 // the power of two at or above its C / VEC vectors), so a head's softmax state
@@ -475,7 +476,7 @@ struct Shape {
   int vec, lph, nch, g;
 };
 bool shape_of(int64_t H, int64_t C, bool al16, bool al8, Shape* s) {
-  if (H < 2 || H > 16 || C < 1 || H * C > 1024) return false;
+  if (H < 1 || H > 16 || C < 1 || H * C > 1024) return false;
   s->vec = C % 4 == 0 && al16 ? 4 : C % 2 == 0 && al8 ? 2 : 1;
   int lph = 1;
   while (lph * s->vec < C) lph *= 2;

@@ -677,10 +677,10 @@ int gr_gat_backward_dst(const int32_t* units, int64_t n_units,
                         float* dd, float* dhs, float* workspace,
                         int64_t n_slots, void* stream);
 
-/* Several heads, one pass over the edges each way (the attention, edge softmax
+/* Attention in one pass over the edges each way (the attention, edge softmax
  * and aggregation of PyG GATConv, grinnder/nn/gat.py:54-61,73, and their
  * backward).  units / fixups / idx / row_idx as gr_gat_forward and
- * gr_gat_backward_src; 2 to 16 heads H of C channels, H * C <= 1024, whose
+ * gr_gat_backward_src; 1 to 16 heads H of C channels, H * C <= 1024, whose
  * lanes (H times the power of two at or above C / 4, or C / 2, or C for rows
  * that 16- or 8-byte accesses do not take) are at most 512, a head's at most 256.
  * Forward: o = O and / or y = O + bias (either may be NULL, not both).  With

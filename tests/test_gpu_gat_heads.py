@@ -21,6 +21,8 @@ CASES = [
     (8, 8, True), (8, 23, True), (8, 32, True), (2, 116, True), (2, 69, True), (4, 49, True),
     (2, 256, True), (2, 512, True), (2, 129, True), (4, 130, True), (16, 64, True),
     (15, 68, True), (6, 6, True), (3, 257, False), (2, 511, False),
+    # one head: 36..64 channels
+    (1, 32, False), (1, 36, True), (1, 48, True), (1, 64, True), (1, 68, False),
 ]
 
 
@@ -61,7 +63,10 @@ def test_heads_match_oracle(gpu, H, C, one_pass, concat, offset):
     assert max_abs_norm_err(b_d.grad, db) <= TOL
     with torch.no_grad():
         again = gat_attention(hs_d, adj, as_d, ad_d, b_d, H, C, concat)
-    assert torch.equal(again, y.detach())
+    if one_pass and offset == 0:  # the same kernel without the backward's state
+        assert torch.equal(again, y.detach())
+    else:
+        assert max_abs_norm_err(again, y.detach()) <= TOL
 
 
 @pytest.mark.parametrize("H,C", [(8, 8), (2, 64), (4, 130)])
