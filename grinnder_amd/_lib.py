@@ -50,6 +50,7 @@ _SIGNATURES = {
                                  _i64, _i64, _P],
     "gr_gcn_aggregate_into": [_P, _i64, _P, _i64, _P, _P, _P, _i64, _P, _P, _i64, _i64, _i64,
                               _P, _i64, _P],
+    "gr_pad_columns": [_i32, _P, _P],
     "gr_gather_rows": [_P, _i64, _i64, _P, _i64, _i64, _P, _i64, _P],
     "gr_scatter_add_rows": [_P, _i64, _i64, _i64, _P, _P, _i64, _i64, _P],
     "gr_column_sum": [_P, _i64, _i64, _i64, _P, _P, _i64, _i64, _P, _P, _i64, _P],
@@ -66,7 +67,7 @@ _SIGNATURES = {
     "gr_xent_forward": [_P, _i64, _i64, _i64, _P, _P, _i32, _P, _P, _i64, _P, _P, _P, _i64, _P],
     "gr_gemm_tn": [_P, _i64, _P, _i64, _i64, _i64, _i64, _f32, _P, _P, _i64, _i64, _P],
     "gr_gemm_nt": [_P, _i64, _P, _i64, _i64, _i64, _i64, _P, _P, _i64, _P],
-    "gr_gemm_nt_split": [_P, _i64, _P, _i64, _i64, _i64, _i64, _P, _P, _i64, _P],
+    "gr_gemm_nt_split": [_P, _i64, _P, _i64, _i32, _i64, _i64, _i64, _P, _P, _i64, _P],
     "gr_gat_scores": [_P, _i64, _i64, _i64, _i64, _i64, _P, _P, _P, _P, _P],
     "gr_gat_row_dot": [_P, _i64, _P, _i64, _i64, _i64, _i64, _P, _P],
     "gr_gat_softmax_stats": [_P, _i64, _P, _i64, _P, _P, _P, _i64, _P, _P, _P, _P, _i64, _P],

@@ -315,16 +315,13 @@ class _GCNLinearAggregatePadded(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x: Tensor, weight: Tensor, bias: Optional[Tensor],
                 plan: DevicePlan) -> Tensor:
-        from torch.nn.functional import pad
-
-        from grinnder_amd.dense import gemm_nt
+        from grinnder_amd.dense import gemm_nt, pad_layer
         d = weight.size(0)
         dp = (d + 3) // 4 * 4
         x = x.contiguous()
-        wp = pad(weight, (0, 0, 0, dp - d))
+        wp, bp = pad_layer(weight, dp, bias)
         with dense_region("fwd", x.size(0), x.size(1), dp):
             z = gemm_nt(x, wp)
-        bp = pad(bias, (0, dp - d)).contiguous() if bias is not None else None
         y = spmm(plan.fwd, plan.idx, plan.val, z, plan.num_dst, bp, name="gcn_fwd")
         ctx.save_for_backward(x, wp)
         ctx.plan = plan
@@ -336,13 +333,11 @@ class _GCNLinearAggregatePadded(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, gy: Tensor):
-        from torch.nn.functional import pad
-
-        from grinnder_amd.dense import gemm_nt_split, gemm_tn
+        from grinnder_amd.dense import gemm_split, gemm_tn, pad_columns
         x, wp = ctx.saved_tensors
         plan: DevicePlan = ctx.plan
         d, dp = ctx.d, wp.size(0)
-        gyp = pad(gy, (0, dp - d)).contiguous()
+        gyp = pad_columns(gy, dp)
         dz = spmm(plan.bwd, plan.row_idx, plan.val_t, gyp, plan.num_src, name="gcn_bwd")
         dx = dw = None
         if ctx.needs_input_grad[0] and ctx.ln_sink is not None:
@@ -350,7 +345,7 @@ class _GCNLinearAggregatePadded(torch.autograd.Function):
             dx = ctx.ln_sink.hand_over(dz, wp, ctx.x_shape)
         elif ctx.needs_input_grad[0]:
             with dense_region("dx", dz.size(0), dp, wp.size(1)):
-                dx = gemm_nt_split(dz, wp.t().contiguous())
+                dx = gemm_split(dz, wp)
         if ctx.needs_input_grad[1]:
             with dense_region("dw", dz.size(0), dp, x.size(1)):
                 dw = gemm_tn(dz, x)[:d]
@@ -533,8 +528,8 @@ class _GCNAggregateLNReLU(torch.autograd.Function):
                                                             bt, ctx.has_bias)
         else:
             if prod is not None:
-                from grinnder_amd.dense import gemm_nt_split
-                gout = gout + gemm_nt_split(prod[0], prod[1].t().contiguous())
+                from grinnder_amd.dense import gemm_split
+                gout = gout + gemm_split(prod[0], prod[1])
             gh, dgamma, dbeta, db = ln_act_backward(gout, h, mean, rstd, g, bt, ctx.has_bias)
         dz = None
         if ctx.sink is not None:
@@ -720,8 +715,18 @@ class _GATAttention(torch.autograd.Function):
                 s_pre: Optional[Tensor] = None, d_pre: Optional[Tensor] = None,
                 sink: Optional[RowDotSink] = None, zsink: Optional[ProjectedSink] = None,
                 token: Optional[Tensor] = None, zx_pre: Optional[Tensor] = None,
-                keep: bool = True) -> Tensor:
-        # keep: a backward may follow (several heads keep its state then).
+                keep: bool = True, trim: int = 0) -> Tensor:
+        # trim: one head padded to `channels`, of which the caller wants the
+        # first `trim`: the output is that view, its gradient padded again.
+        y = _GATAttention._forward(ctx, hs, att_src, att_dst, bias, plan, heads, channels,
+                                   concat, s_pre, d_pre, sink, zsink, zx_pre, keep)
+        ctx.trim = trim
+        return y[:, :trim] if trim else y
+
+    @staticmethod
+    def _forward(ctx, hs, att_src, att_dst, bias, plan, heads, channels, concat, s_pre, d_pre,
+                 sink, zsink, zx_pre, keep):
+        # keep: a backward may follow (the one-pass kernels keep its state then).
         # zsink: hs is the matrix of all partitions' rows ([N, H*C], s_pre
         # [N, H] alike), read in place through zsink.gidx; the backward adds
         # dHs into zsink.dz at zsink.rows.  zx_pre: hs's packed lines
@@ -907,7 +912,7 @@ class _GATAttention(torch.autograd.Function):
         datt_src = column_sum(hs, ds, C)
         datt_dst = column_sum(hs[:B], dd, C)
         return (dhs, datt_src.view(ctx.att_shape), datt_dst.view(ctx.att_shape), db,
-                None, None, None, None, None, None, None, None, None, None, None)
+                None, None, None, None, None, None, None, None, None, None, None, None)
 
     @staticmethod
     def _backward_narrow(ctx, gy: Tensor):
@@ -942,10 +947,13 @@ class _GATAttention(torch.autograd.Function):
         datt_src = column_sum(hs, ds, C)
         datt_dst = column_sum(hs[:B], dd, C)
         return (dhs, datt_src.view(ctx.att_shape), datt_dst.view(ctx.att_shape), db,
-                None, None, None, None, None, None, None, None, None, None, None)
+                None, None, None, None, None, None, None, None, None, None, None, None)
 
     @staticmethod
     def backward(ctx, gy: Tensor):
+        if ctx.trim:
+            from grinnder_amd.dense import pad_columns
+            gy = pad_columns(gy, ctx.shape[1])
         if getattr(ctx, "narrow", False):
             return _GATAttention._backward_narrow(ctx, gy)
         if getattr(ctx, "one_pass", False):
@@ -977,7 +985,7 @@ class _GATAttention(torch.autograd.Function):
         dhs, datt_src, datt_dst = _attention_backward(plan, hs, a_src, a_dst, s, d, alpha_or_m,
                                                       den, go, cdot, H, C, ctx.records, zsink)
         return (dhs, datt_src.view(ctx.att_shape), datt_dst.view(ctx.att_shape), db,
-                None, None, None, None, None, None, None, None, None, None, None)
+                None, None, None, None, None, None, None, None, None, None, None, None)
 
 
 def gat_scores(hs: Tensor, att_src: Tensor, att_dst: Tensor, heads: int, channels: int,
@@ -1014,7 +1022,7 @@ def gat_attention(hs: Tensor, adj: Adjacency, att_src: Tensor, att_dst: Tensor,
                   concat: bool = True,
                   scores: Optional[Tuple[Tensor, Tensor]] = None,
                   rowdot_sink: Optional[RowDotSink] = None,
-                  sink: Optional[ProjectedSink] = None) -> Tensor:
+                  sink: Optional[ProjectedSink] = None, trim: int = 0) -> Tensor:
     """GATConv attention over a bipartite partition adjacency, on the GPU.
 
     hs = lin(x) for all E source rows; destination features are hs[:B].
@@ -1027,9 +1035,14 @@ def gat_attention(hs: Tensor, adj: Adjacency, att_src: Tensor, att_dst: Tensor,
     multiple of 4 in 68..1024 channels), read in place through sink.gidx with
     `scores` = (s of all N rows, d of the partition's rows); the backward adds
     dHs into sink.dz at sink.rows and returns no gradient for hs.
+    `trim`: a head zero-padded to `channels` returns its first `trim` (one
+    head, no sink): y[:, :trim], with the gradient padded in one launch.
     """
     _check_device_tensor("hs", hs)
     plan = adj.device_plan(hs.device)
+    if trim and (heads != 1 or sink is not None or channels % 4 != 0
+                 or not 0 < trim <= channels):
+        raise ValueError("gat_attention: trim is for one padded head without a sink")
     if hs.size(1) != heads * channels:
         raise ValueError(f"hs has {hs.size(1)} features, expected {heads * channels}")
     if sink is not None:
@@ -1051,7 +1064,7 @@ def gat_attention(hs: Tensor, adj: Adjacency, att_src: Tensor, att_dst: Tensor,
         t is not None and t.requires_grad for t in (hs, att_src, att_dst, bias))
     if scores is None:
         return _GATAttention.apply(hs, att_src, att_dst, bias, plan, heads, channels, concat,
-                                   None, None, rowdot_sink, None, None, None, keep)
+                                   None, None, rowdot_sink, None, None, None, keep, trim)
     s, d = scores[0], scores[1]
     if tuple(s.shape) != (plan.num_src, heads) or tuple(d.shape) != (plan.num_dst, heads):
         raise ValueError("gat_attention: scores do not match the adjacency and heads")
@@ -1059,7 +1072,7 @@ def gat_attention(hs: Tensor, adj: Adjacency, att_src: Tensor, att_dst: Tensor,
     if zx is not None and tuple(zx.shape) != (plan.num_src, 32):
         raise ValueError("gat_attention: packed rows do not match the adjacency")
     return _GATAttention.apply(hs, att_src, att_dst, bias, plan, heads, channels, concat, s, d,
-                               rowdot_sink, None, None, zx, keep)
+                               rowdot_sink, None, None, zx, keep, trim)
 
 
 class _GATAttentionLN(torch.autograd.Function):
@@ -1135,8 +1148,8 @@ class _GATAttentionLN(torch.autograd.Function):
                 rowdot=rowdot)
         else:
             if prod is not None:
-                from grinnder_amd.dense import gemm_nt_split
-                gout = gout + gemm_nt_split(prod[0], prod[1].t().contiguous())
+                from grinnder_amd.dense import gemm_split
+                gout = gout + gemm_split(prod[0], prod[1])
             gh, dgamma, dbeta, db = ln_act_backward(gout, h, mean, rstd, g, bt, has_bias,
                                                     ctx.act, shift=ctx.bias, rowdot=rowdot)
         dhs, datt_src, datt_dst = _attention_backward(plan, hs, a_src, a_dst, s, d, m, den, gh,

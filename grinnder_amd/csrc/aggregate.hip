@@ -1455,6 +1455,81 @@ int gr_agg::aggregate_entry(const int32_t* units, int64_t n_units, const int32_t
   return GR_OK;
 }
 
+namespace gr_agg {
+
+// One matrix copied into rows of a multiple of 4 floats, the rest zero.
+struct PadSegment {
+  const float* src;
+  float* dst;
+  int64_t lds, cols;
+  uint32_t quads_row;  // dst row length / 4
+  int64_t first;       // quads before this segment
+};
+struct PadSegments {
+  PadSegment s[4];
+  int n;
+};
+
+// A thread a 16-byte piece of a destination row (grid-stride over all
+// segments): the padded copies of a layer's parameters are one launch instead
+// of a fill and a copy each, and a matrix is written once (200k x 47 -> 48 in
+// 15 us against 12 for torch's fill and 17 for its copy).
+template <typename I>
+__global__ __launch_bounds__(256) void pad_segments_kernel(PadSegments p, int64_t total) {
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < total; t += stride) {
+    int k = 0;
+    while (k + 1 < p.n && t >= p.s[k + 1].first) ++k;
+    const PadSegment& g = p.s[k];
+    const I i = (I)(t - g.first);
+    const I r = i / (I)g.quads_row;
+    const int64_t c = (int64_t)(i - r * (I)g.quads_row) * 4;
+    const float* src = g.src + (int64_t)r * g.lds + c;
+    float4 v;
+    v.x = c + 0 < g.cols ? src[0] : 0.f;
+    v.y = c + 1 < g.cols ? src[1] : 0.f;
+    v.z = c + 2 < g.cols ? src[2] : 0.f;
+    v.w = c + 3 < g.cols ? src[3] : 0.f;
+    reinterpret_cast<float4*>(g.dst)[i] = v;
+  }
+}
+
+}  // namespace gr_agg
+
+extern "C" int gr_pad_columns(int32_t n, const int64_t* segments, void* stream) {
+  gr::clear_error();
+  GR_REQUIRE(n >= 1 && n <= 4 && segments != nullptr, "pad_columns: 1 to 4 segments");
+  gr_agg::PadSegments p;
+  p.n = 0;
+  int64_t total = 0;
+  for (int32_t k = 0; k < n; ++k) {
+    const int64_t* g = segments + 6 * k;
+    const float* src = reinterpret_cast<const float*>(g[0]);
+    float* dst = reinterpret_cast<float*>(g[1]);
+    const int64_t rows = g[2], cols = g[3], lds = g[4], width = g[5];
+    GR_REQUIRE(rows >= 0 && cols >= 0 && lds >= cols && width >= cols && width % 4 == 0 &&
+                   width < (int64_t(1) << 33),
+               "pad_columns: segment %d has a bad shape", (int)k);
+    if (rows == 0 || width == 0) continue;
+    GR_REQUIRE((src || cols == 0) && dst && gr_agg::aligned(dst, 16),
+               "pad_columns: segment %d needs a source and a 16-byte aligned destination", (int)k);
+    p.s[p.n++] = gr_agg::PadSegment{src, dst, lds, cols, (uint32_t)(width / 4), total};
+    total += rows * (width / 4);
+  }
+  if (total == 0) return GR_OK;
+  hipStream_t s = gr::as_stream(stream);
+  const unsigned grid = (unsigned)std::min<int64_t>(8192, (total + 255) / 256);
+  // 32-bit divisions where every index fits (grid strides included).
+  if (total < (int64_t(1) << 31))
+    hipLaunchKernelGGL((gr_agg::pad_segments_kernel<uint32_t>), dim3(grid), dim3(256), 0, s, p,
+                       total);
+  else
+    hipLaunchKernelGGL((gr_agg::pad_segments_kernel<int64_t>), dim3(grid), dim3(256), 0, s, p,
+                       total);
+  GR_HIP_CHECK(hipGetLastError());
+  return GR_OK;
+}
+
 extern "C" int gr_gather_rows(const float* x, int64_t x_rows, int64_t ldx,
                               const int64_t* rows, int64_t n, int64_t dim, float* y,
                               int64_t ldy, void* stream) {

@@ -959,27 +959,35 @@ extern "C" int gr_gemm_nt(const float* a, int64_t lda, const float* b, int64_t l
 // more than rounding; the gradients themselves meet none.
 namespace gr_gemm {
 
-template <int WM, int WN, int MI, int NJ>
-static hipError_t launch_split(const float* a, int64_t lda, const float* b, int64_t ldb,
-                            const float* bias, float* c, int64_t ldc, int64_t m, int n, int k,
-                            bool vec, hipStream_t s) {
+struct SplitArgs {
+  const float* a;
+  int64_t lda;
+  const float* b;
+  int64_t ldb;
+  const float* bias;
+  float* c;
+  int64_t ldc, m;
+  int n, k;
+  bool vec;  // 16-byte rows of A (and of B as [N, K])
+};
+
+template <int WM, int WN, int MI, int NJ, bool KN>
+static hipError_t launch_split(const SplitArgs& g, hipStream_t s) {
   constexpr int BM = WM * MI * 32, BN = WN * NJ * 32;
-  const int tiles_n = (n + BN - 1) / BN;
-  const int64_t grid = ((m + BM - 1) / BM + kXcds - 1) / kXcds * kXcds * tiles_n;
+  const int tiles_n = (g.n + BN - 1) / BN;
+  const int64_t grid = ((g.m + BM - 1) / BM + kXcds - 1) / kXcds * kXcds * tiles_n;
   if (grid > INT32_MAX) return hipErrorInvalidValue;
   const int store =
-      ldc >= (1 << 21) ? 0
-      : n % 4 == 0 && ldc % 4 == 0 && reinterpret_cast<uintptr_t>(c) % 16 == 0 ? 2 : 1;
-  const dim3 g((unsigned)grid), t(WM * WN * 64);
-  if (vec && k % 16 == 0)
-    hipLaunchKernelGGL((gr_bf3::gemm_nt_bf3<WM, WN, MI, NJ, 4, false>), g, t, 0, s, a, lda, b,
-                       ldb, bias, c, ldc, m, n, k, tiles_n, store);
-  else if (vec)
-    hipLaunchKernelGGL((gr_bf3::gemm_nt_bf3<WM, WN, MI, NJ, 4, true>), g, t, 0, s, a, lda, b,
-                       ldb, bias, c, ldc, m, n, k, tiles_n, store);
-  else
-    hipLaunchKernelGGL((gr_bf3::gemm_nt_bf3<WM, WN, MI, NJ, 1, true>), g, t, 0, s, a, lda, b,
-                       ldb, bias, c, ldc, m, n, k, tiles_n, store);
+      g.ldc >= (1 << 21) ? 0
+      : g.n % 4 == 0 && g.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(g.c) % 16 == 0 ? 2 : 1;
+  const dim3 gr((unsigned)grid), t(WM * WN * 64);
+#define GR_SPLIT(V, TAIL)                                                                        \
+  hipLaunchKernelGGL((gr_bf3::gemm_nt_bf3<WM, WN, MI, NJ, V, TAIL, KN>), gr, t, 0, s, g.a, g.lda, \
+                     g.b, g.ldb, g.bias, g.c, g.ldc, g.m, g.n, g.k, tiles_n, store)
+  if (g.vec && g.k % 16 == 0) GR_SPLIT(4, false);
+  else if (g.vec) GR_SPLIT(4, true);
+  else GR_SPLIT(1, true);
+#undef GR_SPLIT
   return hipGetLastError();
 }
 
@@ -994,10 +1002,11 @@ static hipError_t launch_split(const float* a, int64_t lda, const float* b, int6
 //     operands it re-reads (250k x 256 x 1024 643, 128 x 256 655);
 //   64 x 64, or 64 x 32, where those leave CUs without a tile (10k x 64 x 128
 //     7.9, 5k x 128 x 300 11; 128 x 128 10 and 21).
-static hipError_t dispatch_split(const float* a, int64_t lda, const float* b, int64_t ldb,
-                              const float* bias, float* c, int64_t ldc, int64_t m, int n, int k,
-                              bool vec, hipStream_t s) {
-#define GR_NT(...) return launch_split<__VA_ARGS__>(a, lda, b, ldb, bias, c, ldc, m, n, k, vec, s)
+template <bool KN>
+static hipError_t dispatch_split(const SplitArgs& g, hipStream_t s) {
+#define GR_NT(...) return launch_split<__VA_ARGS__, KN>(g, s)
+  const int64_t m = g.m;
+  const int n = g.n, k = g.k;
   const int64_t m128 = (m + 127) / 128, m256 = (m + 255) / 256;
   const int64_t n128 = (n + 127) / 128, n256 = (n + 255) / 256;
   if (n <= 32) {
@@ -1018,21 +1027,24 @@ static hipError_t dispatch_split(const float* a, int64_t lda, const float* b, in
 }  // namespace gr_gemm
 
 extern "C" int gr_gemm_nt_split(const float* a, int64_t lda, const float* b, int64_t ldb,
-                                int64_t m, int64_t n, int64_t k, const float* bias, float* c,
-                                int64_t ldc, void* stream) {
+                                int32_t b_rows_k, int64_t m, int64_t n, int64_t k,
+                                const float* bias, float* c, int64_t ldc, void* stream) {
   using namespace gr_gemm;
   gr::clear_error();
   GR_REQUIRE(m >= 0 && n >= 1 && k >= 1 && n <= (1 << 20) && k <= (1 << 24),
              "gemm_nt_split: bad shape %lld x %lld x %lld", (long long)m, (long long)n,
              (long long)k);
-  GR_REQUIRE(lda >= k && ldb >= k && ldc >= n, "gemm_nt_split: leading dimension too small");
+  GR_REQUIRE(lda >= k && ldb >= (b_rows_k ? n : k) && ldc >= n,
+             "gemm_nt_split: leading dimension too small");
   if (m == 0) return GR_OK;
   GR_REQUIRE(a != nullptr && b != nullptr && c != nullptr, "gemm_nt_split: NULL pointer");
-  const bool vec = k % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 &&
-                   reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
-                   reinterpret_cast<uintptr_t>(b) % 16 == 0;
-  const hipError_t err = dispatch_split(a, lda, b, ldb, bias, c, ldc, m, (int)n, (int)k, vec,
-                                        gr::as_stream(stream));
+  auto rows16 = [&](const float* p, int64_t ld) {
+    return k % 4 == 0 && ld % 4 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+  };
+  const SplitArgs g{a, lda, b, ldb, bias, c, ldc, m, (int)n, (int)k,
+                    rows16(a, lda) && (b_rows_k || rows16(b, ldb))};
+  hipStream_t s = gr::as_stream(stream);
+  const hipError_t err = b_rows_k ? dispatch_split<true>(g, s) : dispatch_split<false>(g, s);
   GR_REQUIRE(err != hipErrorInvalidValue, "gemm_nt_split: too many workgroups for %lld rows",
              (long long)m);
   GR_HIP_CHECK(err);

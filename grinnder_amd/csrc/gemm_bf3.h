@@ -38,7 +38,8 @@ __device__ __forceinline__ float nonfinite(const floatx16& acc, float t) {
 // one barrier a chunk; chunk c + 2 is loaded and chunk c + 1 split and written
 // while chunk c's products run.  The column tiles of one row tile are
 // consecutive workgroups of one XCD, so A is read from HBM once and from that
-// XCD's L2 after.  VEC: 4 with 16-byte rows of A and B, else 1; TAIL: K is
+// XCD's L2 after.  KN: B is [K, N] (dx = dy W from W itself), its pieces read as
+// four rows' elements.  VEC: 4 with 16-byte rows of A (and B), else 1; TAIL: K is
 // not a multiple of 16; store: 2 with 16-byte rows of C, 1 with any rows up to
 // 2^21 floats apart, else 0.  Each output is one wavefront's sum in a fixed order.
 //
@@ -47,7 +48,7 @@ __device__ __forceinline__ float nonfinite(const floatx16& acc, float t) {
 // instructions).  Dealing the split out between the products gained 5% over
 // leaving it in front of them; holding W's pieces from one workgroup to the
 // next would take 1.5 times the LDS there is.
-template <int WM, int WN, int MI, int NJ, int VEC, bool TAIL>
+template <int WM, int WN, int MI, int NJ, int VEC, bool TAIL, bool KN>
 __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_nt_bf3(
     const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
     const float* __restrict__ bias, float* __restrict__ C, int64_t ldc, int64_t M, int N, int K,
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_nt_bf3(
 #pragma unroll
   for (int i = 0; i < SB; ++i) {
     const int row = (tid + i * T) >> 2;
-    pb[i] = Bb + (int64_t)(row < cols ? row : 0) * ldb;
+    pb[i] = KN ? B + n0 + (row < cols ? row : 0) : Bb + (int64_t)(row < cols ? row : 0) * ldb;
   }
   // Loads are unconditional (one basic block a chunk): past the last chunk they
   // re-read it.  With TAIL (K not a multiple of 16) a piece past K reads the
@@ -120,7 +121,16 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_nt_bf3(
         reg[i].w = k + 3 < K ? reg[i].w : 0.f;
       }
     } else {
-      reg[i] = load_piece(pb[i < SA ? 0 : i - SA], k);
+      const float* p = pb[i < SA ? 0 : i - SA];
+      if constexpr (KN) {
+        const int top = K - 1;
+        reg[i].x = p[(int64_t)(TAIL && k + 0 > top ? top : k + 0) * ldb];
+        reg[i].y = p[(int64_t)(TAIL && k + 1 > top ? top : k + 1) * ldb];
+        reg[i].z = p[(int64_t)(TAIL && k + 2 > top ? top : k + 2) * ldb];
+        reg[i].w = p[(int64_t)(TAIL && k + 3 > top ? top : k + 3) * ldb];
+      } else {
+        reg[i] = load_piece(p, k);
+      }
     }
   };
   // Odd rows of A are negated (and their sums again at the end): see the
@@ -232,7 +242,8 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_nt_bf3(
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
         const int col = wn * NJ * 32 + j * 32 + r32;
-        b[j] = in ? Bb[(int64_t)(col < cols ? col : 0) * ldb + k + q] : 0.f;
+        const int64_t at = col < cols ? col : 0;
+        b[j] = !in ? 0.f : KN ? B[(int64_t)(k + q) * ldb + n0 + at] : Bb[at * ldb + k + q];
       }
 #pragma unroll
       for (int i = 0; i < MI; ++i)

@@ -99,17 +99,111 @@ def gemm_tn(a: Tensor, b: Tensor, out: Optional[Tensor] = None, beta: float = 0.
     return out
 
 
-def gemm_nt_split(a: Tensor, b: Tensor, bias: Optional[Tensor] = None,
-                  out: Optional[Tensor] = None) -> Tensor:
-    """gemm_nt on operands split into three bf16 pieces each (24 bits, fp32
-    sums; results no further from float64): faster, with other rounding.  The
-    backward's products run on it; the forward's keep gemm_nt's rounding, so
-    outputs next to an activation's kink keep their side."""
-    return gemm_nt(a, b, bias, out, _entry="gr_gemm_nt_split")
+def _row_strided(t: Tensor) -> Tensor:
+    """t with unit column stride and rows that do not overlap."""
+    if t.stride(1) != 1 or (t.size(0) > 1 and t.stride(0) < t.size(1)):
+        return t.contiguous()
+    return t
+
+
+def gemm_split(a: Tensor, b: Tensor, rows_k: bool = True) -> Tensor:
+    """a b for a [M, K], b [K, N] (rows_k), or a bᵀ for b [N, K]: fp32 device
+    matrices, the operands split into three bf16 pieces each (24 bits, fp32
+    sums; results no further from float64 than gemm_nt's).  The backward's
+    products run on it; the forward's keep gemm_nt's rounding, so outputs next
+    to an activation's kink keep their side."""
+    _check("a", a)
+    _check("b", b)
+    if a.dim() != 2 or b.dim() != 2 or a.size(1) != b.size(0 if rows_k else 1):
+        raise ValueError(f"gemm_split: a {tuple(a.shape)} and b {tuple(b.shape)} do not match")
+    a, b = _row_strided(a), _row_strided(b)
+    m, k = a.shape
+    n = b.size(1 if rows_k else 0)
+    if k == 0:
+        return torch.zeros((m, n), dtype=torch.float32, device=a.device)
+    out = torch.empty((m, n), dtype=torch.float32, device=a.device)
+    if m == 0 or n == 0:
+        return out
+    _lib.call("gr_gemm_nt_split", a.data_ptr(), max(a.stride(0), k), b.data_ptr(),
+              max(b.stride(0), b.size(1)), int(rows_k), m, n, k, None, out.data_ptr(), n,
+              _lib.stream_handle())
+    return out
+
+
+def _pad_launch(segments: list) -> None:
+    """One gr_pad_columns launch over (source, destination, rows, columns,
+    source row stride, destination columns) tuples, flattened."""
+    _lib.call("gr_pad_columns", len(segments) // 6, (ctypes.c_int64 * len(segments))(*segments),
+              _lib.stream_handle())
+
+
+def pad_columns(t: Tensor, width: int) -> Tensor:
+    """A copy of a 2-D fp32 device tensor with zero columns up to `width` (a
+    multiple of 4), written in one pass."""
+    _check("pad_columns: t", t)
+    t = _row_strided(t)
+    rows, cols = t.shape
+    out = torch.empty((rows, width), dtype=torch.float32, device=t.device)
+    _pad_launch([t.data_ptr(), out.data_ptr(), rows, cols, max(t.stride(0), cols), width])
+    return out
+
+
+def pad_layer(weight: Optional[Tensor], width: int, *vectors: Optional[Tensor]) -> list:
+    """[weight with zero rows up to `width` rows (left out when None), each
+    vector zero-padded to `width` in its last dimension (None stays None)], in
+    one launch; width a multiple of 4, at most four tensors, a vector's other
+    dimensions of size 1."""
+    segments, outs = [], []
+    if weight is not None:
+        _check("pad_layer: weight", weight)
+        weight = weight.contiguous()
+        n, din = weight.shape
+        out = torch.empty((width, din), dtype=torch.float32, device=weight.device)
+        segments += [weight.data_ptr(), out.data_ptr(), 1, n * din, n * din, width * din]
+        outs.append(out)
+    keep = []
+    for v in vectors:
+        if v is None:
+            outs.append(None)
+            continue
+        _check("pad_layer: vector", v)
+        v = v.contiguous()
+        keep.append(v)
+        c = v.size(-1)
+        if v.numel() != c:
+            raise ValueError(f"pad_layer: a vector of shape {tuple(v.shape)}")
+        out = torch.empty((*v.shape[:-1], width), dtype=torch.float32, device=v.device)
+        segments += [v.data_ptr(), out.data_ptr(), 1, c, c, width]
+        outs.append(out)
+    if segments:
+        _pad_launch(segments)
+    return outs
+
+
+class _PadLayer(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, width: int, weight: Optional[Tensor], *vectors: Optional[Tensor]):
+        ctx.rows = None if weight is None else weight.size(0)
+        ctx.widths = [None if v is None else v.size(-1) for v in vectors]
+        out = pad_layer(weight, width, *vectors)
+        return tuple(out) if weight is not None else (None, *out)
+
+    @staticmethod
+    def backward(ctx, gw, *gv):
+        return (None, None if gw is None else gw[:ctx.rows],
+                *(None if g is None else g[..., :w] for g, w in zip(gv, ctx.widths)))
+
+
+def pad_layer_grad(weight: Optional[Tensor], width: int, *vectors: Optional[Tensor]) -> tuple:
+    """pad_layer as an autograd function: (weight or None, *vectors) padded."""
+    if not torch.is_grad_enabled():
+        out = pad_layer(weight, width, *vectors)
+        return tuple(out) if weight is not None else (None, *out)
+    return _PadLayer.apply(width, weight, *vectors)
 
 
 def gemm_nt(a: Tensor, b: Tensor, bias: Optional[Tensor] = None,
-            out: Optional[Tensor] = None, _entry: str = "gr_gemm_nt") -> Tensor:
+            out: Optional[Tensor] = None) -> Tensor:
     """C = a bᵀ (+ bias) for a [M, K] and b [N, K] fp32 device matrices with
     unit column stride (rows may be strided) on the matrix cores, or, for a
     short reduction (K <= 64, N >= 64), as a stream of C's rows on the vector
@@ -141,7 +235,7 @@ def gemm_nt(a: Tensor, b: Tensor, bias: Optional[Tensor] = None,
         return out
     if k == 0:
         return out.copy_(bias.expand(m, n) if bias is not None else torch.zeros_like(out))
-    _lib.call(_entry, a.data_ptr(), max(a.stride(0), k), b.data_ptr(),
+    _lib.call("gr_gemm_nt", a.data_ptr(), max(a.stride(0), k), b.data_ptr(),
               max(b.stride(0), k), m, n, k, _lib.ptr(bias), out.data_ptr(),
               max(out.stride(0), n), _lib.stream_handle())
     return out
@@ -181,7 +275,7 @@ class _Linear(torch.autograd.Function):
         rows, dout, din = gy2.size(0), weight.size(0), weight.size(1)
         if ctx.needs_input_grad[0]:
             with dense_region("dx", rows, dout, din):
-                dx = gemm_nt_split(gy2, weight.t().contiguous()).reshape(ctx.in_shape)
+                dx = gemm_split(gy2, weight).reshape(ctx.in_shape)
         if ctx.needs_input_grad[1]:
             with dense_region("dw", rows, dout, din):
                 dw = gemm_tn(gy2, x2)
@@ -247,7 +341,7 @@ class _BiasLNAct(torch.autograd.Function):
                 shift=ctx.bias, rowdot=rowdot)
         else:
             if prod is not None:
-                gout = gout + gemm_nt_split(prod[0], prod[1].t().contiguous())
+                gout = gout + gemm_split(prod[0], prod[1])
             gh, dgamma, dbeta, db = ln_act_backward(gout, h, mean, rstd, g, bt, ctx.has_bias,
                                                     ctx.act, shift=ctx.bias, rowdot=rowdot)
         if ctx.sink is not None:
@@ -324,7 +418,7 @@ class _LinearLNAct(torch.autograd.Function):
         rows, din, dout = x.size(0), x.size(1), w.size(0)
         if ctx.needs_input_grad[0]:
             with dense_region("dx", rows, dout, din):
-                dx = gemm_nt_split(gh, w.t().contiguous())
+                dx = gemm_split(gh, w)
         if ctx.needs_input_grad[1]:
             with dense_region("dw", rows, dout, din):
                 dw = gemm_tn(gh, x)

@@ -19,7 +19,7 @@ from torch import Tensor
 
 from grinnder_amd.aggregation import (KernelTimer, LNProductSink, ProjectedSink, dense_region,
                                       gather_rows, scatter_add_rows)
-from grinnder_amd.dense import OutputRows, gemm_nt, gemm_nt_split, gemm_tn
+from grinnder_amd.dense import OutputRows, gemm_nt, gemm_split, gemm_tn
 from grinnder_amd.loss import masked_cross_entropy
 from grinnder_amd.utils import get_available_host_memory
 
@@ -806,7 +806,7 @@ class ProjectedLayers:
             if ln_sink is not None:
                 return ln_sink.hand_over(dz, wp, consumer.shape)
         with dense_region("dx", hi - lo, w.size(0), w.size(1)):
-            return gemm_nt_split(dz, self._dx_weight(layer, dz.size(1)))
+            return gemm_split(dz, self._dx_weight(layer, dz.size(1)), rows_k=False)
 
     def _padded_weight(self, layer: int, width: int) -> Tensor:
         """The layer's input projection W with zero rows up to `width` (Z's

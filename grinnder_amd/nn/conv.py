@@ -22,7 +22,7 @@ from grinnder_amd.aggregation import (RowDotSink, gat_attention, gat_attention_l
                                       gat_attention_ln_ok, gat_scores, gcn_aggregate,
                                       gcn_linear_aggregate)
 from grinnder_amd.data.adjacency import Adjacency
-from grinnder_amd.dense import bias_ln_act, linear
+from grinnder_amd.dense import bias_ln_act, linear, pad_layer_grad
 
 
 def glorot_(t: Tensor) -> Tensor:
@@ -144,15 +144,13 @@ class GATConv(Module):
             # vectors, so the logits, alpha and the first C output channels
             # are unchanged; the kernels then move 16-byte row vectors.
             pad = (-self.out_channels) % 4
-            w = F.pad(self.lin.weight, (0, 0, 0, pad))
-            a_s = F.pad(self.att_src, (0, pad))
-            a_d = F.pad(self.att_dst, (0, pad))
-            b = F.pad(bias, (0, pad)) if bias is not None else None
+            c = self.out_channels
+            w, a_s, a_d, b = pad_layer_grad(self.lin.weight, c + pad, self.att_src,
+                                            self.att_dst, bias)
             hs = linear(x_src, w, reuse=reuse)
             if keep is not None:
                 keep.append(hs.detach())
-            y = gat_attention(hs, adj, a_s, a_d, b, 1, self.out_channels + pad, self.concat)
-            return y[:, :self.out_channels]
+            return gat_attention(hs, adj, a_s, a_d, b, 1, c + pad, self.concat, trim=c)
         hs = linear(x_src, self.lin.weight, reuse=reuse)
         if keep is not None:
             keep.append(hs.detach())
@@ -190,11 +188,10 @@ class GATConv(Module):
         if pad:
             if sink is not None:
                 raise ValueError("GATConv.attend: a padded head reads gathered rows")
-            b = F.pad(bias, (0, pad)) if bias is not None else None
-            y = gat_attention(self._pad_rows(hs), adj, F.pad(self.att_src, (0, pad)),
-                              F.pad(self.att_dst, (0, pad)), b, 1, self.out_channels + pad,
-                              self.concat, scores)
-            return y[:, :self.out_channels]
+            c = self.out_channels
+            _, a_s, a_d, b = pad_layer_grad(None, c + pad, self.att_src, self.att_dst, bias)
+            return gat_attention(self._pad_rows(hs), adj, a_s, a_d, b, 1, c + pad, self.concat,
+                                 scores, trim=c)
         return gat_attention(hs, adj, self.att_src, self.att_dst, bias, self.heads,
                              self.out_channels, self.concat, scores, rowdot_sink, sink)
 
@@ -231,9 +228,9 @@ class GATConv(Module):
         these rows reads, (s, d, zx), when the head takes them."""
         pad = self._padded()
         if pad:
-            return gat_scores(self._pad_rows(hs), F.pad(self.att_src, (0, pad)),
-                              F.pad(self.att_dst, (0, pad)), 1, self.out_channels + pad,
-                              hs.size(0), packed)
+            width = self.out_channels + pad
+            _, a_s, a_d = pad_layer_grad(None, width, self.att_src, self.att_dst)
+            return gat_scores(self._pad_rows(hs), a_s, a_d, 1, width, hs.size(0), packed)
         return gat_scores(hs, self.att_src, self.att_dst, self.heads, self.out_channels,
                           hs.size(0), packed)
 

@@ -264,6 +264,14 @@ int gr_gcn_aggregate_into(const int32_t* units, int64_t n_units,
                           int64_t ldy, int64_t rows, int64_t dim,
                           float* workspace, int64_t n_slots, void* stream);
 
+/* Up to four matrices [rows, cols] (lds-strided rows) copied into dst [rows,
+ * dst_cols] (contiguous, 16-byte aligned, dst_cols a multiple of 4), the columns
+ * past cols zero, in one launch; segments holds n groups of six: source and
+ * destination address, rows, cols, lds, dst_cols.  For the parameters, gradients and rows of a layer
+ * whose width is not a multiple of 4 (the Linear, attention vectors and bias
+ * inside PyG GCNConv / GATConv, grinnder/nn/gcn.py:53-56, gat.py:54-61). */
+int gr_pad_columns(int32_t n, const int64_t* segments, void* stream);
+
 /* No counterpart in the reference: the row gather from an HBM-resident
  * matrix that the trainer's projected and gathered layers do on the device
  * where the reference gathers halo rows from host buffers
@@ -423,9 +431,10 @@ int gr_gemm_nt(const float* a, int64_t lda, const float* b, int64_t ldb,
                int64_t ldc, void* stream);
 
 /* gr_gemm_nt on split operands (as gr_gemm_tn): the input gradient dx = dy W
- * (B = W^T) of the same Linear. */
+ * of the same Linear.  With b_rows_k != 0 B is [K, N] (W itself, ldb >= n) and
+ * C = A B; else [N, K] as for gr_gemm_nt. */
 int gr_gemm_nt_split(const float* a, int64_t lda, const float* b, int64_t ldb,
-                     int64_t m, int64_t n, int64_t k, const float* bias,
+                     int32_t b_rows_k, int64_t m, int64_t n, int64_t k, const float* bias,
                      float* c, int64_t ldc, void* stream);
 
 /* Dense layer transform with the LayerNorm epilogue in the GEMM accumulators:

@@ -7,7 +7,8 @@ from __future__ import annotations
 import pytest
 import torch
 
-from grinnder_amd.dense import gemm_nt_split, gemm_tn
+from grinnder_amd import _lib
+from grinnder_amd.dense import gemm_split, gemm_tn, pad_columns, pad_layer, pad_layer_grad
 
 pytestmark = pytest.mark.gpu
 
@@ -22,6 +23,17 @@ def gpu():
 def _randn(*shape, seed, dev):
     g = torch.Generator(device=dev).manual_seed(seed)
     return torch.randn(*shape, device=dev, generator=g)
+
+
+def gemm_nt_split(a, b, bias=None, out=None, rows_k=False):
+    """gr_gemm_nt_split with a bias and a strided output."""
+    n = b.size(1 if rows_k else 0)
+    if out is None:
+        out = torch.empty(a.size(0), n, device=a.device)
+    _lib.call("gr_gemm_nt_split", a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
+              int(rows_k), a.size(0), n, a.size(1), _lib.ptr(bias), out.data_ptr(),
+              out.stride(0), _lib.stream_handle())
+    return out
 
 
 def _rel(c, ref):
@@ -51,6 +63,11 @@ def test_gemm_nt_split_tiles_match_fp64(gpu, m, n, k, pad):
     c = gemm_nt_split(a, b, bias, out=out[:m, pad:pad + n])
     ref = a.double() @ b.double().t() + bias.double()
     assert _rel(c, ref) <= _bound(k)
+    # B as [K, N] gives the same sums in the same order.
+    bt = torch.zeros(k, n + pad, device=gpu)[:, pad:]
+    bt.copy_(b.t())
+    assert torch.equal(gemm_nt_split(a, bt, bias, rows_k=True), c)
+    assert torch.equal(gemm_split(a, bt) + bias, c)
     assert bool((out[m] == 7.0).all())  # no row past the last
     if pad:
         assert bool((out[:, 0] == 7.0).all()) and bool((out[:, -1] == 7.0).all())
@@ -125,3 +142,23 @@ def test_products_error_and_bias_against_fp64(gpu):
     ref = x.double().t() @ w.double()
     e = gemm_tn(x, w).double() - ref
     assert float(e.norm() / ref.norm()) <= 1.05 * _rel(x.t() @ w, ref)
+
+
+@pytest.mark.parametrize("rows,cols,width", [(1, 1, 4), (3, 47, 48), (5000, 19, 20), (70, 64, 64),
+                                             (0, 5, 8), (2, 3, 16)])
+def test_pad_columns(gpu, rows, cols, width):
+    """Zero-padded copies equal torch's, strided rows included, and the padded
+    parameters' gradients are the slices."""
+    a = _randn(rows, cols + 3, seed=21, dev=gpu)[:, 1:1 + cols]
+    v = _randn(1, 1, cols, seed=22, dev=gpu)
+    assert torch.equal(pad_columns(a, width), torch.nn.functional.pad(a, (0, width - cols)))
+    assert torch.equal(pad_layer(None, width, v)[0],
+                       torch.nn.functional.pad(v, (0, width - cols)))
+    w = _randn(cols, 7, seed=23, dev=gpu).requires_grad_(True)
+    b = _randn(cols, seed=24, dev=gpu).requires_grad_(True)
+    wp, none, bp = pad_layer_grad(w, width, None, b)
+    assert none is None and torch.equal(wp[:cols], w) and not bool(wp[cols:].any())
+    assert torch.equal(bp[:cols], b) and not bool(bp[cols:].any())
+    g = _randn(width, 7, seed=25, dev=gpu)
+    (wp * g).sum().backward()
+    assert torch.equal(w.grad, g[:cols]) and (b.grad is None or not bool(b.grad.any()))
