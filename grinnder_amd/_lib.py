@@ -155,12 +155,17 @@ def load():
     return _lib
 
 
+_entries = {}
+
+
 def call(name: str, *args) -> None:
     """Calls entry point `name`; raises GrError with the library message on failure."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    fn = _entries.get(name)
+    if fn is None:
+        fn = _entries[name] = getattr(load(), name)
+    rc = fn(*args)
     if rc != 0:
-        msg = lib.gr_last_error().decode(errors="replace")
+        msg = load().gr_last_error().decode(errors="replace")
         raise GrError(f"{name} failed ({rc}): {msg}")
 
 
@@ -172,9 +177,12 @@ def ptr(t) -> int | None:
 
 
 def stream_handle(stream=None) -> int | None:
-    """Raw hipStream_t of a torch stream (the current stream by default)."""
+    """Raw hipStream_t of a torch stream (the current stream by default).
+
+    The default asks torch's C++ side for the handle: building the Stream
+    object takes about 4 us, once for every kernel launched."""
     if stream is None:
-        stream = torch.cuda.current_stream()
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
     return stream.cuda_stream
 
 

@@ -37,6 +37,9 @@ class KernelRecord:
         return self.start.elapsed_time(self.end)
 
 
+_UNTIMED = contextlib.nullcontext()
+
+
 class KernelTimer:
     """Records HIP events around every aggregation pass (and, as "dense_*"
     regions with their flop counts, every dense product) while active.
@@ -78,12 +81,17 @@ class KernelTimer:
         return self._pool.pop() if self._pool else torch.cuda.Event(enable_timing=True)
 
     @staticmethod
-    @contextlib.contextmanager
     def region(name: str, nbytes: int, edges: int, dim: int, flops: int = 0):
+        """A context that times what is launched inside it, while a timer is
+        active; one shared empty context otherwise."""
         timer = KernelTimer.active
         if timer is None:
-            yield
-            return
+            return _UNTIMED
+        return KernelTimer._timed(timer, name, nbytes, edges, dim, flops)
+
+    @staticmethod
+    @contextlib.contextmanager
+    def _timed(timer: "KernelTimer", name: str, nbytes: int, edges: int, dim: int, flops: int):
         start = timer._event()
         end = timer._event()
         start.record()

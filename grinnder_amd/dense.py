@@ -17,6 +17,7 @@ afterwards, and LayerNorm + ELU after a GAT layer.
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional, Tuple
 
 import torch
@@ -63,6 +64,7 @@ def output_block(dest: Optional[OutputRows], rows: int, dim: int, device) -> Ten
     return t
 
 
+@functools.lru_cache(maxsize=256)
 def gemm_tn_splits(m: int, n: int, k: int) -> Tuple[int, int]:
     """Default K split count and workspace floats of ``gemm_tn`` for a shape."""
     splits = ctypes.c_int64(0)

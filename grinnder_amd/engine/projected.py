@@ -176,7 +176,12 @@ class ProjectedLayers:
         blocks torch's caching allocator holds unused (an earlier epoch's
         kept graphs and temporaries, which the allocator hands out again)."""
         free, _ = torch.cuda.mem_get_info(self.device)
-        return free + torch.cuda.memory_reserved(self.device) - torch.cuda.memory_allocated(self.device)
+        # The nested form: the flat one builds and sorts some 150 entries a call.
+        stats = torch.cuda.memory_stats_as_nested_dict(self.device)
+        if not stats:  # nothing allocated yet
+            return free
+        return (free + stats["reserved_bytes"]["all"]["current"]
+                - stats["allocated_bytes"]["all"]["current"])
 
     def _plan_projection(self) -> Dict[int, Tensor]:
         """Layers this epoch runs projected, with their input projection W:
