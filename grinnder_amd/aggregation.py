@@ -599,24 +599,17 @@ def _gat_heads_ok(hs: Tensor, heads: int, channels: int) -> bool:
     """Whether the attention runs in one online-softmax pass each way
     (gr_gat_heads_forward / _backward).
 
-    Several heads: where their lanes fit, heads times the power of two at or
-    above a head's vectors, at most 512 lanes (256 a head); wider rows take the
-    general kernels.  One head: 36..128 channels on 16-byte rows, where the
+    Several heads: always.  One head: 36..128 channels on 16-byte rows, where the
     one-head kernels run rows of up to 32 edges and longer ones as two launches
     (us forward and backward / forward alone, theirs first: 48 channels over 2M
     edges, 100k rows 327/133 and 255/102, 128 channels 447/170 and 400/155).
     Up to 32 channels half the lanes would idle (28: 306/79 and 261/107, 176/48
     and 246/50 for 1M edges, 30k rows), and past 128 a wavefront has one edge
     slot either way (164: 306/121 and 338/134 there)."""
-    rows = hs.data_ptr() | 4 * hs.stride(0)
     if heads == 1:
-        return channels % 4 == 0 and 32 < channels <= 64 and rows % 16 == 0
-    if not 2 <= heads <= 16:
-        return False
-    vec = (4 if channels % 4 == 0 and rows % 16 == 0
-           else 2 if channels % 2 == 0 and rows % 8 == 0 else 1)
-    lanes = 1 << ((channels + vec - 1) // vec - 1).bit_length()
-    return lanes <= 256 and heads * lanes <= 512 and heads * channels <= 1024
+        return (channels % 4 == 0 and 32 < channels <= 64
+                and (hs.data_ptr() | 4 * hs.stride(0)) % 16 == 0)
+    return 2 <= heads <= 16 and heads * channels <= 1024
 
 
 def _attention_backward(plan: DevicePlan, hs: Tensor, a_src: Tensor, a_dst: Tensor, s: Tensor,

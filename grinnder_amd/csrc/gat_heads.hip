@@ -3,7 +3,7 @@
 // grinnder/nn/gat.py:54-61,69-78).
 //
 // Lanes are laid out by head: head h owns LPH consecutive lane positions (LPH
-// the power of two at or above its C / VEC vectors), so a head's softmax state
+// the power of two at or above its C / 4 vectors), so a head's softmax state
 // is held by its own lanes, its dot products are reduced over an aligned lane
 // group, and no loop runs over the heads.  A wavefront takes one plan unit
 // (row, edge range, slot) at a time; for narrow rows (up to 32 lane positions)
@@ -43,14 +43,16 @@ __device__ __forceinline__ int64_t wave_id() {
   return (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 }
 
+// Four floats at any 4-byte boundary: one access, as aligned ones (a head's
+// rows start anywhere when its channels are not a multiple of 4; 8 heads of 27
+// and 2 of 95 took 2 to 4 times as long with 4-byte accesses).
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+
 template <int VEC>
 __device__ __forceinline__ void ld(const float* __restrict__ p, float (&r)[VEC]) {
   if constexpr (VEC == 4) {
-    const float4 t = *reinterpret_cast<const float4*>(p);
+    const float4u t = *reinterpret_cast<const float4u*>(p);
     r[0] = t.x; r[1] = t.y; r[2] = t.z; r[3] = t.w;
-  } else if constexpr (VEC == 2) {
-    const float2 t = *reinterpret_cast<const float2*>(p);
-    r[0] = t.x; r[1] = t.y;
   } else {
     r[0] = *p;
   }
@@ -58,22 +60,25 @@ __device__ __forceinline__ void ld(const float* __restrict__ p, float (&r)[VEC])
 
 template <int VEC>
 __device__ __forceinline__ void st(float* __restrict__ p, const float (&r)[VEC]) {
-  if constexpr (VEC == 4) *reinterpret_cast<float4*>(p) = make_float4(r[0], r[1], r[2], r[3]);
-  else if constexpr (VEC == 2) *reinterpret_cast<float2*>(p) = make_float2(r[0], r[1]);
+  if constexpr (VEC == 4) *reinterpret_cast<float4u*>(p) = float4u{r[0], r[1], r[2], r[3]};
   else *p = r[0];
 }
 
 // A lane's place in chunk ch of a row: head, feature and whether it holds any
-// (lanes that do not read head 0's first vector and count as 0).
+// (lanes that do not read head 0's first vector and count as 0).  The last
+// vector of a head whose channels are not a multiple of 4 ends with the head:
+// its first `dup` features are its neighbour's too.  Both hold and store the
+// same values for them; sums over the head leave them out here.
 struct Place {
-  int head, feat;
+  int head, feat, dup;
   bool ok, lead;  // lead: the first lane of its head
 };
 template <int VEC>
 __device__ __forceinline__ Place place(int p, int lph, int H, int C) {
   const int h = p / lph, v = p & (lph - 1);
   const bool ok = h < H && v * VEC < C;
-  return Place{ok ? h : 0, ok ? h * C + v * VEC : 0, ok, ok && v == 0};
+  const int c = v * VEC + VEC <= C ? v * VEC : C - VEC;
+  return Place{ok ? h : 0, ok ? h * C + c : 0, ok ? v * VEC - c : VEC, ok, ok && v == 0};
 }
 
 // t[u][ch] summed over the lanes of its head, for U edges at once: one uniform
@@ -319,10 +324,11 @@ __global__ __launch_bounds__(256) void gat_heads_bwd_dst(
       t[0][ch] = t[1][ch] = 0.f;
 #pragma unroll
       for (int q = 0; q < VEC; ++q) {
-        t[0][ch] = fmaf(g[q], a[q], t[0][ch]);
-        t[1][ch] = fmaf(g[q], b[q], t[1][ch]);
+        if (q >= pl[ch].dup) {
+          t[0][ch] = fmaf(g[q], a[q], t[0][ch]);
+          t[1][ch] = fmaf(g[q], b[q], t[1][ch]);
+        }
       }
-      if (!pl[ch].ok) t[0][ch] = t[1][ch] = 0.f;
     }
     head_sums<2, NCH>(t, lph);
 #pragma unroll
@@ -367,7 +373,7 @@ __global__ __launch_bounds__(256) void gat_heads_bwd_src(
 #pragma unroll
     for (int q = 0; q < VEC; ++q) {
       acc[ch][q] = 0.f;
-      if (!pl[ch].ok) hsj[ch][q] = 0.f;
+      hsj[ch][q] = q >= pl[ch].dup ? hsj[ch][q] : 0.f;
     }
   }
   int inext = w.y < w.z ? row_idx[min(w.y + lane, w.z - 1)] : 0;
@@ -470,27 +476,26 @@ __global__ __launch_bounds__(256) void gat_heads_bwd_fixup(
 
 // ------------------------------------------------------------ dispatch --
 
-// Vector width, lanes per head and chunks of a row; false if the row takes
-// more than eight chunks of 64 lanes (then gat.hip's general kernels run).
+// Vector width, lanes per head, chunks of a row and lanes a slot.  Heads of at
+// least 4 channels take 16-byte accesses; H * C <= 1024 then needs at most 512
+// lanes.
 struct Shape {
   int vec, lph, nch, g;
 };
-bool shape_of(int64_t H, int64_t C, bool al16, bool al8, Shape* s) {
+bool shape_of(int64_t H, int64_t C, Shape* s) {
   if (H < 1 || H > 16 || C < 1 || H * C > 1024) return false;
-  s->vec = C % 4 == 0 && al16 ? 4 : C % 2 == 0 && al8 ? 2 : 1;
+  s->vec = C >= 4 ? 4 : 1;
   int lph = 1;
   while (lph * s->vec < C) lph *= 2;
   const int lanes = (int)H * lph;
   s->lph = lph;
   s->nch = 1;
   while (64 * s->nch < lanes) s->nch *= 2;
-  // A head of more than 64 lanes spans whole chunks: at most four.
-  if (s->nch > 8 || lph > 256) return false;
+  if (s->nch > 8 || lph > 256) return false;  // a head spans at most four chunks
   s->g = lanes <= 16 ? 16 : lanes <= 32 ? 32 : 64;
   return true;
 }
 
-inline bool al(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
 inline unsigned blocks_for(int64_t waves) { return (unsigned)((waves + 3) / 4); }
 
 // Edges in flight a lane, by chunks and vector width: at most 32 registers of
@@ -517,8 +522,9 @@ using namespace gr_gath;
 #define GR_HEADS(CALL)                                  \
   do {                                                  \
     if (sh.vec == 4) GR_HEADS_SHAPES(4, CALL);          \
-    else if (sh.vec == 2) GR_HEADS_SHAPES(2, CALL);     \
-    else GR_HEADS_SHAPES(1, CALL);                      \
+    else if (sh.g == 16) CALL(1, 16, 1);                \
+    else if (sh.g == 32) CALL(1, 32, 1);                \
+    else CALL(1, 64, 1);                                \
   } while (0)
 
 extern "C" int gr_gat_heads_workspace(int64_t H, int64_t C, int32_t with_state,
@@ -541,12 +547,7 @@ extern "C" int gr_gat_heads_forward(const int32_t* units, int64_t n_units, const
   GR_REQUIRE(n_units >= 0 && n_fix >= 0 && n_slots >= 0, "gat_heads_forward: negative count");
   GR_REQUIRE(ldh >= H * C, "gat_heads_forward: leading dimension too small");
   const bool with_bias = y != nullptr;
-  const uintptr_t both = (with_bias ? reinterpret_cast<uintptr_t>(bias) |
-                                          reinterpret_cast<uintptr_t>(y)
-                                    : 0) |
-                         reinterpret_cast<uintptr_t>(hs) | reinterpret_cast<uintptr_t>(o) |
-                         reinterpret_cast<uintptr_t>(nrow) | reinterpret_cast<uintptr_t>(ws);
-  GR_REQUIRE(shape_of(H, C, ldh % 4 == 0 && both % 16 == 0, ldh % 2 == 0 && both % 8 == 0, &sh),
+  GR_REQUIRE(shape_of(H, C, &sh),
              "gat_heads_forward: %lld heads of %lld channels", (long long)H, (long long)C);
   GR_REQUIRE((state != nullptr) == (nrow != nullptr) && (o != nullptr || y != nullptr) &&
                  (!with_bias || bias != nullptr),
@@ -598,12 +599,7 @@ extern "C" int gr_gat_heads_backward(const int32_t* units, int64_t n_units,
   GR_REQUIRE(n_units >= 0 && n_fix >= 0 && n_slots >= 0 && n_dst >= 0,
              "gat_heads_backward: negative count");
   GR_REQUIRE(ldh >= H * C, "gat_heads_backward: leading dimension too small");
-  const uintptr_t all = reinterpret_cast<uintptr_t>(hs) | reinterpret_cast<uintptr_t>(go) |
-                        reinterpret_cast<uintptr_t>(o) | reinterpret_cast<uintptr_t>(nrow) |
-                        reinterpret_cast<uintptr_t>(att_src) |
-                        reinterpret_cast<uintptr_t>(att_dst) |
-                        reinterpret_cast<uintptr_t>(dhs) | reinterpret_cast<uintptr_t>(ws);
-  GR_REQUIRE(shape_of(H, C, ldh % 4 == 0 && all % 16 == 0, ldh % 2 == 0 && all % 8 == 0, &sh),
+  GR_REQUIRE(shape_of(H, C, &sh),
              "gat_heads_backward: %lld heads of %lld channels", (long long)H, (long long)C);
   GR_REQUIRE(n_units <= int64_t(INT32_MAX) * 4, "gat_heads_backward: too many units");
   const int64_t stride = pad4((int)(H * C)) + pad4((int)H);

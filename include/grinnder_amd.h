@@ -689,9 +689,8 @@ int gr_gat_backward_dst(const int32_t* units, int64_t n_units,
 /* Attention in one pass over the edges each way (the attention, edge softmax
  * and aggregation of PyG GATConv, grinnder/nn/gat.py:54-61,73, and their
  * backward).  units / fixups / idx / row_idx as gr_gat_forward and
- * gr_gat_backward_src; 1 to 16 heads H of C channels, H * C <= 1024, whose
- * lanes (H times the power of two at or above C / 4, or C / 2, or C for rows
- * that 16- or 8-byte accesses do not take) are at most 512, a head's at most 256.
+ * gr_gat_backward_src; 1 to 16 heads H of C channels, H * C <= 1024, rows at any
+ * 4-byte boundary.
  * Forward: o = O and / or y = O + bias (either may be NULL, not both).  With
  * state ([rows, H] float4) and nrow ([rows, H*C]) it also keeps what the
  * backward needs: (d, m, den, S) and N = sum of alpha Hs over the edges with

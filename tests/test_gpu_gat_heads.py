@@ -1,6 +1,6 @@
 """Several attention heads in one pass (csrc/gat_heads.hip) against the oracle:
-every lane layout (heads and channels around powers of two, 16-, 8- and 4-byte
-rows, one to eight chunks a row, edge slots), split and empty rows, and the
+every lane layout (heads and channels around powers of two, rows at any 4-byte
+boundary, one to eight chunks a row, edge slots), split and empty rows, and the
 forward without a backward."""
 
 from __future__ import annotations
@@ -20,7 +20,7 @@ CASES = [
     (2, 1, True), (16, 1, True), (2, 2, True), (3, 5, True), (5, 16, True), (7, 12, True),
     (8, 8, True), (8, 23, True), (8, 32, True), (2, 116, True), (2, 69, True), (4, 49, True),
     (2, 256, True), (2, 512, True), (2, 129, True), (4, 130, True), (16, 64, True),
-    (15, 68, True), (6, 6, True), (3, 257, False), (2, 511, False),
+    (15, 68, True), (6, 6, True), (3, 257, True), (2, 511, True), (5, 3, True), (16, 63, True),
     # one head: 36..64 channels
     (1, 32, False), (1, 36, True), (1, 48, True), (1, 64, True), (1, 68, False),
 ]
