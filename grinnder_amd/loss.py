@@ -6,8 +6,9 @@ Replaces the loss and metric code of the reference trainer:
 ``compute_micro_f1`` (grinnder/utils.py:24-44) for the val / test rows.  One
 HIP pass (``gr_xent_forward``) reads the logits once and produces the loss,
 the accuracy counts and the gradient of the train-row nll sum; the backward
-only scales that gradient, so the logits may be released after the forward
-(the partitioned trainer frees the last layer's output right away).
+(``gr_xent_backward``) only scales that gradient, so the logits may be released
+after the forward (the partitioned trainer frees the last layer's output right
+away).
 """
 
 from __future__ import annotations
@@ -21,6 +22,7 @@ from grinnder_amd import _lib
 
 TRAIN, VAL, TEST = 1, 2, 4
 _STATS = 7            # per-workgroup partial statistics of gr_xent_forward
+_TRAIN_WORDS = 4      # 64-bit words of a workgroup's train rows' bits
 _ROWS_PER_BLOCK = 256
 
 
@@ -45,7 +47,7 @@ class _MaskedCrossEntropy(torch.autograd.Function):
         loss = torch.empty((), dtype=torch.float32, device=dev)
         stats = torch.empty(6, dtype=torch.int64, device=dev)
         nblk = max(1, (rows + _ROWS_PER_BLOCK - 1) // _ROWS_PER_BLOCK)
-        ws = torch.empty(nblk * _STATS, dtype=torch.float64, device=dev)
+        ws = torch.empty(nblk * (_STATS + _TRAIN_WORDS), dtype=torch.float64, device=dev)
         need_grad = ctx.needs_input_grad[0]
         grad = torch.empty((rows, classes), dtype=torch.float32, device=dev) if need_grad \
             else None
@@ -54,18 +56,36 @@ class _MaskedCrossEntropy(torch.autograd.Function):
                   classes, loss.data_ptr(), stats.data_ptr(), ws.data_ptr(), ws.numel(),
                   _lib.stream_handle())
         if need_grad:
-            ctx.save_for_backward(grad, stats)
+            ctx.save_for_backward(grad, stats, ws)
         ctx.mean = mean
+        ctx.set_materialize_grads(False)
         ctx.mark_non_differentiable(stats)
         return loss, stats
 
     @staticmethod
     def backward(ctx, gloss: Tensor, _gstats):
-        grad, stats = ctx.saved_tensors
+        if gloss is None:
+            return None, None, None, None
+        grad, stats, ws = ctx.saved_tensors
+        n_train = stats.data_ptr() if ctx.mean else None
         scale = gloss.to(torch.float32)
-        if ctx.mean:
-            scale = scale / stats[0].clamp(min=1).to(torch.float32)
-        return grad * scale, None, None, None
+        rows, classes = grad.shape
+        out = torch.empty_like(grad)
+        train = ws.data_ptr() + 8 * _STATS * max(1, (rows + _ROWS_PER_BLOCK - 1) // _ROWS_PER_BLOCK)
+        try:
+            at = scale.data_ptr()
+        except RuntimeError:  # batched by vmap (is_grads_batched)
+            at = None
+        if at is None or (scale.requires_grad and torch.is_grad_enabled()):
+            # The scale as torch operations, which vmap and a second
+            # differentiation see.
+            one = torch.ones((), dtype=torch.float32, device=grad.device)
+            _lib.call("gr_xent_backward", grad.data_ptr(), rows, classes, train, one.data_ptr(),
+                      n_train, out.data_ptr(), _lib.stream_handle())
+            return out * scale, None, None, None
+        _lib.call("gr_xent_backward", grad.data_ptr(), rows, classes, train, at, n_train,
+                  out.data_ptr(), _lib.stream_handle())
+        return out, None, None, None
 
 
 def masked_cross_entropy(logits: Tensor, labels: Tensor, codes: Tensor,
