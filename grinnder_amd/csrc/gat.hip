@@ -128,6 +128,87 @@ __global__ __launch_bounds__(256) void gat_scores_kernel(const float* __restrict
   }
 }
 
+// The same with several heads of 4, 8, .. 256 channels on 16-byte rows: a head
+// is a group of LPH = C / 4 lanes (a power of two), its sums are reduced within
+// the group, and G lanes hold a row, 64 / G rows a wavefront and step.  The
+// kernel above sums over the whole wavefront once per head and result, 12
+// H exchanges a row, which bound it at 8 heads; here they are 2 log2(LPH), in
+// the same order (the lanes outside a head added zeros), so the results are the
+// same, and the read of the rows bounds it: 8 heads
+// of 32 over 200k rows 83 -> 33 us (6.2 TB/s), 8 of 8 over 50k 28 -> 4.8 us.
+template <int G, int NCH, int U>
+__global__ __launch_bounds__(256) void gat_scores_heads(const float* __restrict__ hs, int64_t ldh,
+                                                        int64_t n_src, int64_t n_dst, int H,
+                                                        int lph_log2,
+                                                        const float* __restrict__ att_src,
+                                                        const float* __restrict__ att_dst,
+                                                        float* __restrict__ s,
+                                                        float* __restrict__ d) {
+  constexpr int RPW = 64 / G;
+  static_assert(RPW == 1 || NCH == 1, "rows side by side hold one chunk");
+  const int lane = threadIdx.x & 63;
+  const int slot = lane / G, li = lane % G;
+  const int nv = H << lph_log2;  // 16-byte vectors of a row
+  int fld[NCH], hd[NCH];
+  float as[NCH][4], ad[NCH][4];
+#pragma unroll
+  for (int ch = 0; ch < NCH; ++ch) {
+    const int v = ch * 64 + li;
+    const bool lead = v < nv && (v & ((1 << lph_log2) - 1)) == 0;
+    fld[ch] = v < nv ? 4 * v : 0;
+    hd[ch] = lead ? v >> lph_log2 : -1;  // the head that this lane stores
+    ld<4>(att_src + fld[ch], as[ch]);
+    ld<4>(att_dst + fld[ch], ad[ch]);
+  }
+  const int64_t step = (int64_t)gridDim.x * 4 * RPW * U;
+  for (int64_t r0 = wave_id() * RPW * U; r0 < n_src; r0 += step) {
+    float x[U][NCH][4], t[2 * U * NCH];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int64_t r = r0 + k * RPW + slot;
+#pragma unroll
+      for (int ch = 0; ch < NCH; ++ch)
+        ld<4>(hs + (r < n_src ? r : n_src - 1) * ldh + fld[ch], x[k][ch]);
+    }
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+#pragma unroll
+      for (int ch = 0; ch < NCH; ++ch) {
+        float ps = 0.f, pd = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          ps = fmaf(x[k][ch][q], as[ch][q], ps);
+          pd = fmaf(x[k][ch][q], ad[ch][q], pd);
+        }
+        t[2 * (k * NCH + ch)] = ps;
+        t[2 * (k * NCH + ch) + 1] = pd;
+      }
+    // Over the head's lanes: one uniform branch for all sums.
+#define GR_EACH(N)                                               \
+  _Pragma("unroll") for (int k = 0; k < 2 * U * NCH; ++k) t[k] = gr_wave::group_sum<N>(t[k])
+    switch (lph_log2) {
+      case 1: GR_EACH(2); break;
+      case 2: GR_EACH(4); break;
+      case 3: GR_EACH(8); break;
+      case 4: GR_EACH(16); break;
+      case 5: GR_EACH(32); break;
+      case 6: GR_EACH(64); break;
+      default: break;  // a head is one lane
+    }
+#undef GR_EACH
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int64_t r = r0 + k * RPW + slot;
+#pragma unroll
+      for (int ch = 0; ch < NCH; ++ch) {
+        if (hd[ch] < 0 || r >= n_src) continue;
+        s[r * H + hd[ch]] = t[2 * (k * NCH + ch)];
+        if (r < n_dst) d[r * H + hd[ch]] = t[2 * (k * NCH + ch) + 1];
+      }
+    }
+  }
+}
+
 // cdot[i,h] = <a[i,h,:], b[i,h,:]> (the backward's c_i = <GO_i, O_i>): the
 // same row walk as the scores kernel with a second row in place of the
 // attention vectors.
@@ -1725,6 +1806,27 @@ extern "C" int gr_gat_scores(const float* hs, int64_t ldh, int64_t n_src, int64_
     const int64_t waves = (n_src + u - 1) / u;
     return dim3((unsigned)std::min<int64_t>(4096, (waves + 3) / 4));
   };
+  const int64_t lph = channels / 4;
+  if (heads > 1 && al && channels % 4 == 0 && lph <= 64 && (lph & (lph - 1)) == 0) {
+    // Heads of a power-of-two number of 16-byte vectors up to one wavefront:
+    // never slower than the loop over the heads, with the same results.  Other
+    // widths would sum in another order, and a logit within rounding of
+    // LeakyReLU's kink could change its slope.
+    int log2 = 0;
+    while ((1 << log2) < lph) ++log2;
+    const int64_t nv = heads * lph;  // at most 256 (check_heads)
+#define GR_SH(G, N, U)                                                                      \
+  hipLaunchKernelGGL((gat_scores_heads<G, N, U>), grid(U * (64 / G)), dim3(256), 0, st, hs, ldh, \
+                     n_src, n_dst, H, log2, att_src, att_dst, s, d)
+    if (nv <= 16) GR_SH(16, 1, 4);
+    else if (nv <= 32) GR_SH(32, 1, 4);
+    else if (nv <= 64) GR_SH(64, 1, 4);
+    else if (nv <= 128) GR_SH(64, 2, 2);
+    else GR_SH(64, 4, 1);
+#undef GR_SH
+    GR_HIP_CHECK(hipGetLastError());
+    return GR_OK;
+  }
 #define GR_SC(V, N, U)                                                                   \
   hipLaunchKernelGGL((gat_scores_kernel<V, N, U>), grid(U), dim3(256), 0, st, hs, ldh, n_src, \
                      n_dst, H, C, att_src, att_dst, s, d)
