@@ -412,15 +412,35 @@ static hipError_t launch_nt(const float* a, int64_t lda, const float* b, int64_t
 // one slice ahead, explicit instruction interleaving and 64 x 128 wavefront
 // tiles were each measured and gained nothing; double-buffered LDS pays only
 // in the 16-k, 4-waves-per-SIMD form above.
+//
+// Few rows: with fewer tiles than CUs the chip idles and a tile's serial k
+// loop is the time, so they are cut to 64 rows (64 columns past 64).  Same
+// blocks and k order, so the same bits.  us, large and 64-row tiles: 10k x 64 x
+// 128 15.1 and 6.3, 50k-row 64 x 256 29.5 and 27.3, 10k x 256 x 256 25.7 and
+// 19.9, 5k x 128 x 300 27.3 and 11.7.  The line is one tile a CU, where the small
+// tiles still gain (60k x 48 x 256 23.4 and 22.2); at 470 to 940 tiles they lose up
+// to 15% (40k x 256 x 100 32.4 and 37.9).
+constexpr int64_t kFewTiles = 256;
 template <int VA, int VB>
 static hipError_t dispatch_nt(const float* a, int64_t lda, const float* b, int64_t ldb,
                               const float* bias, float* c, int64_t ldc, int64_t m, int n, int k,
                               hipStream_t s) {
 #define GR_NT(MI, NJ, WMW, KS, BLK, ...) \
   return launch_nt<VA, VB, MI, NJ, WMW, KS, BLK, ##__VA_ARGS__>(a, lda, b, ldb, bias, c, ldc, m, n, k, s)
+  // Workgroups of a tile; below kFewTiles the 64-row tiles.
+  auto few = [&](int tm, int tn) {
+    return ((m + tm - 1) / tm) * ((n + tn - 1) / tn) < kFewTiles;
+  };
   if (n > 64) {
+    if (few(128, 128)) GR_NT(1, 1, 2, 32, 32);
     if (k <= 256) GR_NT(2, 2, 2, 16, 32, 4, true);
     GR_NT(2, 2, 2, 32, 32);
+  }
+  if (few(256, 64)) {
+    if (n > 48) GR_NT(1, 4, 4, 32, 16);
+    if (n > 32) GR_NT(1, 3, 4, 32, 16);
+    if (n > 16) GR_NT(1, 2, 4, 32, 16);
+    GR_NT(1, 1, 4, 32, 16);
   }
   if (n > 48) GR_NT(4, 4, 4, 16, 16, 1, true);
   if (n > 32) GR_NT(4, 3, 4, 32, 16);
