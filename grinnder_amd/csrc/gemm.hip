@@ -416,7 +416,7 @@ static hipError_t launch_nt(const float* a, int64_t lda, const float* b, int64_t
 // Few rows: with fewer tiles than CUs the chip idles and a tile's serial k
 // loop is the time, so they are cut to 64 rows (64 columns past 64).  Same
 // blocks and k order, so the same bits.  us, large and 64-row tiles: 10k x 64 x
-// 128 15.1 and 6.3, 50k-row 64 x 256 29.5 and 27.3, 10k x 256 x 256 25.7 and
+// 128 15.1 and 6.3, 40k x 64 x 256 27.7 and 21.0, 10k x 256 x 256 25.7 and
 // 19.9, 5k x 128 x 300 27.3 and 11.7.  The line is one tile a CU, where the small
 // tiles still gain (60k x 48 x 256 23.4 and 22.2); at 470 to 940 tiles they lose up
 // to 15% (40k x 256 x 100 32.4 and 37.9).
