@@ -68,7 +68,9 @@ __device__ __forceinline__ void st(float* __restrict__ p, const float (&r)[VEC])
 // (lanes that do not read head 0's first vector and count as 0).  The last
 // vector of a head whose channels are not a multiple of 4 ends with the head:
 // its first `dup` features are its neighbour's too.  Both hold and store the
-// same values for them; sums over the head leave them out here.
+// same values for them; sums over the head leave them out here, by a select and
+// not by a factor of 0, which an infinity or NaN of head 0 would turn into NaN
+// in a lane of another head.
 struct Place {
   int head, feat, dup;
   bool ok, lead;  // lead: the first lane of its head
@@ -371,10 +373,7 @@ __global__ __launch_bounds__(256) void gat_heads_bwd_src(
     sj[ch] = s[j * H + pl[ch].head];
     dsl[ch] = 0.f;
 #pragma unroll
-    for (int q = 0; q < VEC; ++q) {
-      acc[ch][q] = 0.f;
-      hsj[ch][q] = q >= pl[ch].dup ? hsj[ch][q] : 0.f;
-    }
+    for (int q = 0; q < VEC; ++q) acc[ch][q] = 0.f;
   }
   int inext = w.y < w.z ? row_idx[min(w.y + lane, w.z - 1)] : 0;
   for (int b = w.y; b < w.z; b += 64) {
@@ -400,7 +399,8 @@ __global__ __launch_bounds__(256) void gat_heads_bwd_src(
         for (int ch = 0; ch < NCH; ++ch) {
           t[u][ch] = 0.f;
 #pragma unroll
-          for (int q = 0; q < VEC; ++q) t[u][ch] = fmaf(g[u][ch][q], hsj[ch][q], t[u][ch]);
+          for (int q = 0; q < VEC; ++q)
+            t[u][ch] = q >= pl[ch].dup ? fmaf(g[u][ch][q], hsj[ch][q], t[u][ch]) : t[u][ch];
         }
       head_sums<U, NCH>(t, lph);
 #pragma unroll

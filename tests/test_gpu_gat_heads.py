@@ -88,3 +88,49 @@ def test_heads_extreme_logits(gpu, H, C):
     reads[rows[col == 399]] = True
     got = gat_attention(bad.to(gpu), adj, a_s.to(gpu), a_d.to(gpu), bias.to(gpu), H, C).cpu()
     assert bool(got[~reads].isfinite().all()) and bool(got[reads].isnan().all())
+
+
+@pytest.mark.parametrize("H,C", [(3, 12), (7, 20), (8, 27), (4, 36), (2, 69), (5, 3), (3, 5),
+                                 (4, 130), (3, 341), (8, 8)])
+@pytest.mark.parametrize("head", [0, -1])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_a_nonfinite_gradient_stays_in_its_head(gpu, H, C, head, value):
+    """An infinite or NaN output gradient of one head leaves the other heads'
+    gradients as they were, bit for bit, also where lanes of a head hold
+    nothing (they read head 0's first vector) or share features with a
+    neighbour; in its own head NaN appears where float64 gives it."""
+    rows = 260
+    rowptr, col, adj, hs, a_s, a_d, _, gy = _inputs(H, C, True)
+    head = head % H
+    bad = gy.view(rows, H, C).clone()
+    if head == 0:
+        bad[::9, 0, 0] = value
+    else:
+        bad[::9, head, C - 1] = value  # a shared vector's part when C % 4 != 0
+    bad = bad.view(rows, H * C)
+
+    def grads(g):
+        t = [x.to(gpu).requires_grad_(True) for x in (hs, a_s, a_d)]
+        y = gat_attention(t[0], adj, t[1], t[2], None, H, C, True)
+        return [x.reshape(-1, H, C).cpu() for x in torch.autograd.grad(y, t, g.to(gpu))]
+
+    clean, got = grads(gy), grads(bad)
+    others = [h for h in range(H) if h != head]
+    for a, b in zip(got, clean):
+        assert torch.equal(a[:, others], b[:, others])
+    # The head itself, in float64 and the kernels' order: c = <G, O>, edge
+    # gradients alpha (<G, Hs> - c).  Rows past the destinations, which get no
+    # part from a destination's own logit.
+    o, alpha, tpre = oracle.gat_forward(rowptr, col, hs, H, C, a_s, a_d, None, True)
+    row = torch.repeat_interleave(torch.arange(rows), rowptr[1:] - rowptr[:-1])
+    g = bad.view(rows, H, C)[:, head].double()
+    h64 = hs.view(-1, H, C)[:, head].double()
+    c = (g * torch.as_tensor(o).view(rows, H, C)[:, head]).sum(1)
+    alpha, slope = (torch.as_tensor(t)[:, head] for t in (alpha, tpre))
+    ge = alpha * ((g[row] * h64[col]).sum(1) - c[row])
+    ds = torch.zeros(hs.size(0), dtype=torch.float64)
+    ds.index_add_(0, col, torch.where(slope > 0, ge, 0.2 * ge))
+    want = torch.zeros_like(h64).index_add_(0, col, alpha[:, None] * g[row])
+    want += ds[:, None] * a_s[0, head].double()
+    assert torch.equal(got[0][rows:, head].isnan(), want[rows:].isnan())
+    assert bool(want[rows:].isnan().any()) and not bool(want[rows:].isnan().all())
