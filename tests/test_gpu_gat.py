@@ -401,3 +401,45 @@ def test_gat_attention_ln_matches_attention_then_epilogue(gpu, C, longs):
         assert err <= TOL, name
     if longs == 0:
         assert torch.equal(res[0][0], res[1][0])
+
+
+@pytest.mark.parametrize("C", [10, 27, 47, 70, 130])
+@pytest.mark.parametrize("add_bias", [True, False])
+def test_odd_width_output_changed_in_place(gpu, C, add_bias):
+    """A one-head layer whose width is no multiple of 4 (it runs zero-padded)
+    gives an output that may be changed in place: with a bias and more than 24
+    channels the gradients are those of the same operations out of place.
+    Where the backward reads the output itself (up to 24 channels, or no bias)
+    the change is found out, not taken for the layer's output."""
+    from grinnder_amd.nn import GATConv
+    rowptr, col, val = random_bipartite(150, 200, 6, seed=C, long_rows=1, long_len=700)
+    adj = Adjacency(rowptr, col, val, (150, 200))
+    torch.manual_seed(C)
+    conv = GATConv(33, C, heads=1, add_self_loops=False).to(gpu)
+    x = torch.randn(200, 33, device=gpu)
+    mask = torch.rand(150, C, device=gpu) < 0.3
+
+    def grads(in_place):
+        y = conv((x, x[:150]), adj, add_bias=add_bias)
+        assert y.shape == (150, C) and y.stride() == ((C + 3) // 4 * 4, 1)
+        if in_place:
+            y.mul_(2.0).masked_fill_(mask, 0.0)
+            torch.nn.functional.relu_(y[:, 1:])
+        else:
+            y = (2.0 * y).masked_fill(mask, 0.0)
+            y = torch.cat([y[:, :1], torch.relu(y[:, 1:])], 1)
+        params = [conv.lin.weight, conv.att_src, conv.att_dst]
+        return [y.detach(), *torch.autograd.grad(y.pow(2).sum(), params)]
+
+    want = grads(False)
+    if add_bias and C > 24:
+        for a, b in zip(grads(True), want):
+            assert torch.equal(a, b)
+    else:
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            grads(True)
+    with torch.no_grad():
+        y = conv((x, x[:150]), adj, add_bias=add_bias)
+        y.mul_(2.0).masked_fill_(mask, 0.0)
+        torch.nn.functional.relu_(y[:, 1:])
+    assert torch.equal(y, want[0])
