@@ -65,6 +65,8 @@ _SIGNATURES = {
     "gr_linear_ln_act": [_P, _i64, _i64, _i64, _P, _i64, _P, _P, _P, _f32, _i32, _P, _P, _P, _P,
                          _P],
     "gr_xent_forward": [_P, _i64, _i64, _i64, _P, _P, _i32, _P, _P, _i64, _P, _P, _P, _i64, _P],
+    "gr_xent_forward_train": [_P, _i64, _i64, _i64, _P, _P, _i32, _P, _i64, _P, _P, _P, _P, _i64,
+                              _P],
     "gr_xent_backward": [_P, _i64, _i64, _P, _P, _P, _P, _P],
     "gr_gemm_tn": [_P, _i64, _P, _i64, _i64, _i64, _i64, _f32, _P, _P, _i64, _i64, _P],
     "gr_gemm_nt": [_P, _i64, _P, _i64, _i64, _i64, _i64, _P, _P, _i64, _P],

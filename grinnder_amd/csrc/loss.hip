@@ -13,7 +13,8 @@
 // val / test rows outside [0, C) are counted and reported, not read.
 // Gradient rows: g[r, c] = exp(x_c - m) / sum - [c == y] on train rows (0 if
 // the label is out of range), i.e. d(sum of train nll)/dx, the backward of
-// log_softmax + NLL; other rows are not written.
+// log_softmax + NLL; other rows are 0, or, where the train rows' bits are kept
+// for xent_backward to tell them apart, not written.
 //
 // 1M rows of 47 classes, 60% train: forward 136 us, backward 62 and four small
 // launches when every row's gradient was written, with a second exponential
@@ -198,7 +199,8 @@ __global__ __launch_bounds__(256) void xent_rows_narrow(const float* __restrict_
       count[3] += __popcll(__ballot(lead && ok && (mk[u] & 4) && hit));
       count[4] += __popcll(__ballot(lead && ok && (mk[u] & 4)));
       count[5] += __popcll(__ballot(lead && mk[u] != 0 && !ok));
-      if (grad != nullptr && in && (mk[u] & 1)) {
+      const bool train = mk[u] & 1;
+      if (grad != nullptr && in && (train || bits == nullptr)) {
         const float inv = 1.f / sum;
         float* g = grad + r * ldg;
 #pragma unroll
@@ -206,7 +208,7 @@ __global__ __launch_bounds__(256) void xent_rows_narrow(const float* __restrict_
           float q[V];
 #pragma unroll
           for (int i = 0; i < V; ++i)
-            q[i] = ok ? v[u][k][i] * inv - (start[k] + i == yc ? 1.f : 0.f) : 0.f;
+            q[i] = ok && train ? v[u][k][i] * inv - (start[k] + i == yc ? 1.f : 0.f) : 0.f;
           if (k + 1 == R && (l + k * G) * V >= C) continue;  // nothing of its own
           if constexpr (V == 4) {
             *reinterpret_cast<float4u*>(g + start[k]) = float4u{q[0], q[1], q[2], q[3]};
@@ -266,10 +268,11 @@ __global__ __launch_bounds__(256) void xent_rows_wide(const float* __restrict__ 
     const uint8_t mk = mask[r];
     const int64_t y = labels[r];
     const bool ok_label = y >= 0 && y < C;
-    if (grad != nullptr && (mk & 1)) {
+    const bool train = mk & 1;
+    if (grad != nullptr && (train || bits == nullptr)) {
       float* g = grad + r * ldg;
       for (int c = lane; c < C; c += 64)
-        g[c] = ok_label ? expf(row[c] - lse) - (c == (int)y ? 1.f : 0.f) : 0.f;
+        g[c] = ok_label && train ? expf(row[c] - lse) - (c == (int)y ? 1.f : 0.f) : 0.f;
     }
     if (lane == 0) {
       if (lse_out != nullptr) lse_out[r] = lse;
@@ -372,13 +375,14 @@ __global__ __launch_bounds__(256) void xent_finish(const double* __restrict__ pa
 
 }  // namespace gr_loss
 
-extern "C" int gr_xent_forward(const float* logits, int64_t ld, int64_t rows, int64_t classes,
-                               const int64_t* labels, const uint8_t* mask, int32_t mean,
-                               float* lse, float* grad, int64_t ldg, float* loss,
-                               int64_t* stats, double* workspace, int64_t workspace_doubles,
-                               void* stream) {
-  using namespace gr_loss;
-  gr::clear_error();
+namespace gr_loss {
+
+// bits: NULL, or where the train rows' bits go; the gradient's other rows are
+// then left to gr_xent_backward.
+static int forward(const float* logits, int64_t ld, int64_t rows, int64_t classes,
+                   const int64_t* labels, const uint8_t* mask, int32_t mean, float* lse,
+                   float* grad, int64_t ldg, uint64_t* bits, float* loss, int64_t* stats,
+                   double* workspace, int64_t workspace_doubles, void* stream) {
   GR_REQUIRE(rows >= 0 && classes >= 1 && classes <= (1 << 24) && ld >= classes,
              "xent_forward: bad shape (%lld rows, %lld classes, ld %lld)", (long long)rows,
              (long long)classes, (long long)ld);
@@ -391,9 +395,6 @@ extern "C" int gr_xent_forward(const float* logits, int64_t ld, int64_t rows, in
              "%lld needed", (long long)workspace_doubles, (long long)(nblk * kStats));
   hipStream_t s = gr::as_stream(stream);
   const int c = (int)classes;
-  // Room behind the partials for the train rows' bits: kept for the backward.
-  uint64_t* bits = workspace_doubles >= nblk * (kStats + kRowsPerBlock / 64)
-                       ? reinterpret_cast<uint64_t*>(workspace + nblk * kStats) : nullptr;
   // With rows == 0 the single workgroup writes zero partials.
 #define GR_XENT(G, R, V, U)                                                             \
   hipLaunchKernelGGL((xent_rows_narrow<G, R, V, U>), dim3((unsigned)nblk), dim3(256), 0, s, \
@@ -412,6 +413,30 @@ extern "C" int gr_xent_forward(const float* logits, int64_t ld, int64_t rows, in
                      stats);
   GR_HIP_CHECK(hipGetLastError());
   return GR_OK;
+}
+
+}  // namespace gr_loss
+
+extern "C" int gr_xent_forward(const float* logits, int64_t ld, int64_t rows, int64_t classes,
+                               const int64_t* labels, const uint8_t* mask, int32_t mean,
+                               float* lse, float* grad, int64_t ldg, float* loss,
+                               int64_t* stats, double* workspace, int64_t workspace_doubles,
+                               void* stream) {
+  gr::clear_error();
+  return gr_loss::forward(logits, ld, rows, classes, labels, mask, mean, lse, grad, ldg, nullptr,
+                          loss, stats, workspace, workspace_doubles, stream);
+}
+
+extern "C" int gr_xent_forward_train(const float* logits, int64_t ld, int64_t rows,
+                                     int64_t classes, const int64_t* labels, const uint8_t* mask,
+                                     int32_t mean, float* grad, int64_t ldg, uint64_t* train,
+                                     float* loss, int64_t* stats, double* workspace,
+                                     int64_t workspace_doubles, void* stream) {
+  gr::clear_error();
+  GR_REQUIRE(rows == 0 || (grad != nullptr && train != nullptr),
+             "xent_forward_train: NULL output");
+  return gr_loss::forward(logits, ld, rows, classes, labels, mask, mean, nullptr, grad, ldg, train,
+                          loss, stats, workspace, workspace_doubles, stream);
 }
 
 extern "C" int gr_xent_backward(const float* grad, int64_t rows, int64_t classes,

@@ -4,7 +4,7 @@ Replaces the loss and metric code of the reference trainer:
 ``F.cross_entropy(out[train], y[train], reduction="sum"|"mean")``
 (grinnder/engine/trainer.py:709-721 per partition, :430-453 fast path) and
 ``compute_micro_f1`` (grinnder/utils.py:24-44) for the val / test rows.  One
-HIP pass (``gr_xent_forward``) reads the logits once and produces the loss,
+HIP pass (``gr_xent_forward_train``) reads the logits once and produces the loss,
 the accuracy counts and the gradient of the train-row nll sum; the backward
 (``gr_xent_backward``) only scales that gradient, so the logits may be released
 after the forward (the partitioned trainer frees the last layer's output right
@@ -22,7 +22,7 @@ from grinnder_amd import _lib
 
 TRAIN, VAL, TEST = 1, 2, 4
 _STATS = 7            # per-workgroup partial statistics of gr_xent_forward
-_TRAIN_WORDS = 4      # 64-bit words of a workgroup's train rows' bits
+_TRAIN_WORDS = 4      # 64-bit words of a workgroup's train rows' bits, after the partials
 _ROWS_PER_BLOCK = 256
 
 
@@ -51,12 +51,16 @@ class _MaskedCrossEntropy(torch.autograd.Function):
         need_grad = ctx.needs_input_grad[0]
         grad = torch.empty((rows, classes), dtype=torch.float32, device=dev) if need_grad \
             else None
-        _lib.call("gr_xent_forward", logits.data_ptr(), logits.stride(0), rows, classes,
-                  labels.data_ptr(), codes.data_ptr(), int(mean), None, _lib.ptr(grad),
-                  classes, loss.data_ptr(), stats.data_ptr(), ws.data_ptr(), ws.numel(),
-                  _lib.stream_handle())
+        at = (logits.data_ptr(), logits.stride(0), rows, classes, labels.data_ptr(),
+              codes.data_ptr(), int(mean))
+        out = (loss.data_ptr(), stats.data_ptr(), ws.data_ptr(), nblk * _STATS,
+               _lib.stream_handle())
         if need_grad:
+            _lib.call("gr_xent_forward_train", *at, grad.data_ptr(), classes,
+                      ws.data_ptr() + 8 * nblk * _STATS, *out)
             ctx.save_for_backward(grad, stats, ws)
+        else:
+            _lib.call("gr_xent_forward", *at, None, None, 0, *out)
         ctx.mean = mean
         ctx.set_materialize_grads(False)
         ctx.mark_non_differentiable(stats)

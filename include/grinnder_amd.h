@@ -389,22 +389,30 @@ int gr_bias_ln_act(const float* z, int64_t ldz, const float* bias,
  * label outside [0, classes)} (the caller raises on the last), lse[r] =
  * log-sum-exp of row r (may be NULL), and, when grad != NULL, the gradient of
  * the train-row nll sum, grad[r, c] = softmax(x_r)_c - [c == y_r] on train
- * rows (0 where the label is out of range; ldg-strided); other rows are not
- * written.  gr_xent_backward scales it by dL/dloss (and 1 / train rows for the
- * mean) and fills them in.  Sums are reduced in a fixed order in double.
- * workspace: 7 * n doubles, n = max(1, ceil(rows / 256)); given 11 * n, the
- * 64-bit words from word 7 * n on receive the train rows' bits (bit r % 64 of
- * word r / 64). */
+ * rows (0 where the label is out of range) and 0 elsewhere (ldg-strided); the
+ * caller scales it by dL/dloss (and 1 / train rows for the mean).  Sums are
+ * reduced in a fixed order in double.
+ * workspace: 7 * max(1, ceil(rows / 256)) doubles. */
 int gr_xent_forward(const float* logits, int64_t ld, int64_t rows,
                     int64_t classes, const int64_t* labels, const uint8_t* mask,
                     int32_t mean, float* lse, float* grad, int64_t ldg,
                     float* loss, int64_t* stats, double* workspace,
                     int64_t workspace_doubles, void* stream);
 
+/* The forward of gr_xent_backward: gr_xent_forward (without lse) that leaves
+ * grad's rows outside the train set unwritten and the train rows' bits in
+ * `train` (4 * max(1, ceil(rows / 256)) words; bit r % 64 of word r / 64).
+ * Neither may be NULL unless rows == 0. */
+int gr_xent_forward_train(const float* logits, int64_t ld, int64_t rows,
+                          int64_t classes, const int64_t* labels, const uint8_t* mask,
+                          int32_t mean, float* grad, int64_t ldg, uint64_t* train,
+                          float* loss, int64_t* stats, double* workspace,
+                          int64_t workspace_doubles, void* stream);
+
 /* out = grad * *gloss (/ max(*n_train, 1) when n_train, a device int64, is not
- * NULL) on the rows whose bit in `train` (as gr_xent_forward leaves them) is
- * set, 0 on the others, whose grad is not read: the backward of
- * gr_xent_forward's loss.  grad and out are dense [rows, classes]. */
+ * NULL) on the rows whose bit in `train` is set, 0 on the others, whose grad is
+ * not read: the backward of gr_xent_forward_train's loss.  grad and out are
+ * dense [rows, classes]. */
 int gr_xent_backward(const float* grad, int64_t rows, int64_t classes,
                      const uint64_t* train, const float* gloss,
                      const int64_t* n_train,
