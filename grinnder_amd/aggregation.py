@@ -1074,8 +1074,11 @@ def gat_attention(hs: Tensor, adj: Adjacency, att_src: Tensor, att_dst: Tensor,
     # backward: sliced outside the function they share the saved tensor's
     # version, so that a change in place is seen.
     inner = trim if bias is not None and channels > 24 else 0
+    # Any input that asks for a gradient brings a backward, the scores (which
+    # get none) among them.
     keep = torch.is_grad_enabled() and any(
-        t is not None and t.requires_grad for t in (hs, att_src, att_dst, bias))
+        t is not None and t.requires_grad
+        for t in (hs, att_src, att_dst, bias, *(scores or ())))
     if scores is None:
         y = _GATAttention.apply(hs, att_src, att_dst, bias, plan, heads, channels, concat,
                                 None, None, rowdot_sink, None, None, None, keep, inner)

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import oracle
-from grinnder_amd.aggregation import _gat_heads_ok, gat_attention
+from grinnder_amd.aggregation import _gat_heads_ok, gat_attention, gat_scores
 from grinnder_amd.data.adjacency import Adjacency
 from tests.graphs import TOL, max_abs_norm_err, random_bipartite
 
@@ -134,3 +134,22 @@ def test_a_nonfinite_gradient_stays_in_its_head(gpu, H, C, head, value):
     want += ds[:, None] * a_s[0, head].double()
     assert torch.equal(got[0][rows:, head].isnan(), want[rows:].isnan())
     assert bool(want[rows:].isnan().any()) and not bool(want[rows:].isnan().all())
+
+
+@pytest.mark.parametrize("H,C", [(8, 8), (2, 256), (1, 48)])
+def test_backward_when_only_the_scores_ask_for_a_gradient(gpu, H, C):
+    """Frozen rows and parameters with precomputed scores that require a
+    gradient: the backward runs and gives the scores none, and the gradients
+    of a row leaf beside such scores are those with detached ones."""
+    _, _, adj, hs, a_s, a_d, _, gy = (t if not torch.is_tensor(t) else t.to(gpu)
+                                      for t in _inputs(H, C, True))
+    s, d = gat_scores(hs, a_s, a_d, H, C, gy.size(0))
+    s, d = s.requires_grad_(True), d.requires_grad_(True)
+    y = gat_attention(hs, adj, a_s, a_d, None, H, C, scores=(s, d))
+    assert y.requires_grad
+    y.backward(gy)
+    assert s.grad is None and d.grad is None
+    leaf = hs.clone().requires_grad_(True)
+    got = [torch.autograd.grad(gat_attention(leaf, adj, a_s, a_d, None, H, C, scores=sc), leaf,
+                               gy)[0] for sc in ((s, d), (s.detach(), d.detach()))]
+    assert torch.equal(got[0], got[1])
