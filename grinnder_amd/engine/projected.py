@@ -271,8 +271,8 @@ class ProjectedLayers:
         # autograd graph until its backward, which then skips the recompute
         # (an aggregation pass and a gather of Z per partition); the last
         # layer's loss is then taken from the kept logits, which no longer
-        # go through host memory.  What a graph holds is bounded by the
-        # gathered rows, three [N, d_out] tensors and one float per edge.
+        # go through host memory.  What a graph holds is the model's to say
+        # (kept_floats).
         self._keep = set()
         if self.model.training:
             sum_e = sum(g.expanded_sizes)
@@ -281,10 +281,10 @@ class ProjectedLayers:
             for layer in sorted(plan):
                 if layer + 1 not in self._xin and layer != last:
                     continue
-                d = plan[layer].size(0)
+                per_row, per_out, per_edge = self.model.kept_floats(layer)
                 if free is None:
                     free = self._free_device_memory()
-                need = 4 * (sum_e * d + 3 * n * d + nnz)
+                need = 4 * (sum_e * per_row + n * per_out + nnz * per_edge)
                 if need + (8 << 30) > free:
                     continue
                 free -= need

@@ -62,6 +62,16 @@ class GriNNderModel(torch.nn.Module):
         past W's rows at zero)."""
         return self.input_projection(layer).size(0)
 
+    def kept_floats(self, layer: int) -> tuple:
+        """(per gathered row of Z, per output row, per edge) floats that the
+        autograd graph of forward_projected(layer, ...) holds, its input and
+        output included: what a partitioned trainer counts with when it
+        decides whether the graphs of all partitions fit in device memory
+        until their backward.  The default: the gathered rows, three tensors
+        of their width and one float per edge."""
+        width = self.projected_width(layer)
+        return width, 3 * width, 1
+
     def projected_sink_ok(self, layer: int) -> bool:
         """Whether forward_projected(layer, ...) accepts a sink."""
         return False

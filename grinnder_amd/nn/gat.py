@@ -93,6 +93,20 @@ class GAT(GriNNderModel):
         conv = self.convs[layer]
         return conv.heads * conv.out_channels + conv._padded()
 
+    def kept_floats(self, layer: int) -> tuple:
+        """By the attention kernels that run the layer (gat_attention): one
+        head of at most 24 channels keeps its rows' packed 32-float lines and
+        C + 4 floats of state a row; several heads, or one of up to 64 channels,
+        O, the backward's second row sum and a 16-byte record per head beside
+        the layer's output before and after its activation; a wider head O and
+        those two."""
+        w, heads = self.projected_width(layer), self.convs[layer].heads
+        if heads == 1 and w <= 24:
+            return w + 33, 3 * w + 8, 0
+        if heads > 1 or 32 < w <= 64:
+            return w + heads, 4 * w + 5 * heads + 2, 0
+        return w + 1, 3 * w + 6, 1
+
     def projected_sink_ok(self, layer: int) -> bool:
         """Z read in place for one head of 68..1024 channels (a multiple of
         4): the attention gathers each edge's source row of Z directly and

@@ -11,6 +11,7 @@ import torch
 import oracle
 from grinnder_amd.aggregation import _gat_heads_ok, gat_attention, gat_scores
 from grinnder_amd.data.adjacency import Adjacency
+from grinnder_amd.nn import GAT
 from tests.graphs import TOL, max_abs_norm_err, random_bipartite
 
 pytestmark = pytest.mark.gpu
@@ -153,3 +154,35 @@ def test_backward_when_only_the_scores_ask_for_a_gradient(gpu, H, C):
     got = [torch.autograd.grad(gat_attention(leaf, adj, a_s, a_d, None, H, C, scores=sc), leaf,
                                gy)[0] for sc in ((s, d), (s.detach(), d.detach()))]
     assert torch.equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("heads,C,norm,last", [
+    (8, 32, False, False), (8, 32, True, False), (1, 48, True, False), (1, 47, False, True),
+    (1, 256, True, False), (1, 100, False, False), (1, 100, True, False), (1, 20, False, True),
+    (16, 8, False, False)])
+def test_kept_floats_covers_what_a_layers_graph_holds(gpu, heads, C, norm, last):
+    """The floats that a trainer counts for a kept forward graph against the
+    device memory it holds: never less, beyond the allocator's rounding, and
+    not a third more."""
+    E, B = 200_000, 160_000
+    g = torch.Generator().manual_seed(C)
+    adj = Adjacency(torch.arange(B + 1) * 4, torch.randint(0, E, (4 * B,), generator=g), None,
+                    (B, E))
+    model = (GAT(4, 16, C, 2, heads=1, dropout=0.0) if last else
+             GAT(8, C, 4, 2, heads=heads, dropout=0.0, norm=norm)).to(gpu).train()
+    layer = int(last)
+    z = torch.randn(E, model.projected_width(layer), device=gpu)
+    z[:, heads * C:] = 0.0
+    s, d = model.projected_scores(layer, z)
+    z.requires_grad_(True)
+    model.forward_projected(layer, z, adj, scores=(s, d[:B]))  # builds the plan
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    out = model.forward_projected(layer, z, adj, scores=(s, d[:B]))
+    held = torch.cuda.memory_allocated() - before + 4 * (z.numel() + s.numel())
+    assert out.requires_grad
+    per_row, per_out, per_edge = model.kept_floats(layer)
+    count = 4 * (E * per_row + B * per_out + 4 * B * per_edge)
+    print(f"held {held / 1e6:.1f} MB, counted {count / 1e6:.1f} MB", flush=True)
+    assert held <= count + (8 << 20)  # the allocator leaves up to 1 MB at a large tensor's end
+    assert count <= 4 / 3 * held
