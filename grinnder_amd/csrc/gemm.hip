@@ -449,8 +449,8 @@ static hipError_t dispatch_nt(const float* a, int64_t lda, const float* b, int64
 #undef GR_NT
 }
 
-// Products with a short reduction (k <= 64: a layer's input gradient
-// dZ W through a narrow layer) whose operands are not 16-byte aligned.  A
+// Products with a short reduction (k <= 64: a layer with few input features)
+// whose operands are not 16-byte aligned.  A
 // wavefront owns 128 columns (2 adjacent ones per lane, their rows of B held
 // in registers) and a run of SK_ROWS rows of C; lane kk holds A[r][kk],
 // loaded SK_PD rows ahead, and row r's k values reach every lane by
@@ -939,7 +939,7 @@ extern "C" int gr_gemm_nt(const float* a, int64_t lda, const float* b, int64_t l
     err = dispatch_resident(a, lda, b, ldb, bias, c, ldc, m, (int)n, (int)k, s);
   } else if (k <= 64 && n >= 64 && !(va && vb)) {
     // Short reduction with rows of A or B that 16-byte loads cannot take
-    // (k or ld not a multiple of 4, as for a 19- or 47-wide gradient): on the
+    // (k or ld not a multiple of 4, as for 19 or 47 input features): on the
     // vector units as a stream of C's rows (gemm_nt_short_k), 1.3-1.6x faster
     // than the matrix-core kernel with 4-byte loads.  With aligned rows the
     // matrix cores stay faster (1.0 against 1.9 ms for 2.45M x 256 x 48).
@@ -976,7 +976,8 @@ extern "C" int gr_gemm_nt(const float* a, int64_t lda, const float* b, int64_t l
 // and closer to float64.  The forward product stays on gr_gemm_nt: its results
 // meet the ReLU and LeakyReLU kinks, and an output within rounding of one that
 // changed side would change the elementwise input gradients behind it by far
-// more than rounding; the gradients themselves meet none.
+// more than rounding; the gradients themselves meet none.  The package reads W
+// as it lies ([K, N]); the [N, K] form serves C callers that hold W transposed.
 namespace gr_gemm {
 
 struct SplitArgs {

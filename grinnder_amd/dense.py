@@ -108,27 +108,26 @@ def _row_strided(t: Tensor) -> Tensor:
     return t
 
 
-def gemm_split(a: Tensor, b: Tensor, rows_k: bool = True) -> Tensor:
-    """a b for a [M, K], b [K, N] (rows_k), or a bᵀ for b [N, K]: fp32 device
-    matrices, the operands split into three bf16 pieces each (24 bits, fp32
-    sums; results no further from float64 than gemm_nt's).  The backward's
-    products run on it; the forward's keep gemm_nt's rounding, so outputs next
-    to an activation's kink keep their side."""
+def gemm_split(a: Tensor, b: Tensor) -> Tensor:
+    """a b for a [M, K], b [K, N]: fp32 device matrices, the operands split into
+    three bf16 pieces each (24 bits, fp32 sums; results no further from float64
+    than gemm_nt's).  The backward's products run on it; the forward's keep
+    gemm_nt's rounding, so outputs next to an activation's kink keep their
+    side."""
     _check("a", a)
     _check("b", b)
-    if a.dim() != 2 or b.dim() != 2 or a.size(1) != b.size(0 if rows_k else 1):
+    if a.dim() != 2 or b.dim() != 2 or a.size(1) != b.size(0):
         raise ValueError(f"gemm_split: a {tuple(a.shape)} and b {tuple(b.shape)} do not match")
     a, b = _row_strided(a), _row_strided(b)
     m, k = a.shape
-    n = b.size(1 if rows_k else 0)
+    n = b.size(1)
     if k == 0:
         return torch.zeros((m, n), dtype=torch.float32, device=a.device)
     out = torch.empty((m, n), dtype=torch.float32, device=a.device)
     if m == 0 or n == 0:
         return out
     _lib.call("gr_gemm_nt_split", a.data_ptr(), max(a.stride(0), k), b.data_ptr(),
-              max(b.stride(0), b.size(1)), int(rows_k), m, n, k, None, out.data_ptr(), n,
-              _lib.stream_handle())
+              max(b.stride(0), n), 1, m, n, k, None, out.data_ptr(), n, _lib.stream_handle())
     return out
 
 

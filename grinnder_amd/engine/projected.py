@@ -105,7 +105,6 @@ class ProjectedLayers:
         # W padded with zero rows to Z's width, per projected layer whose Z is
         # wider than W's rows (formed once per epoch: W changes between).
         self._wpad: Dict[int, Tensor] = {}
-        self._wtdx: Dict[int, Tensor] = {}
         # HBM buffers of dL/dx for the gathered layers above layer 0 (layers
         # in self._xin that run neither projected nor in place), by layer.
         self._gxbufs: Dict[int, Tensor] = {}
@@ -211,7 +210,6 @@ class ProjectedLayers:
         self._out_room = False
         self._merge_room = False
         self._wpad = {}
-        self._wtdx = {}
         if (self._fast or cfg.mode != "grinnder" or cfg.project_first == "off"
                 or self.cache is not None
                 or (self._pid_start, self._pid_end) != (0, g.num_parts)):
@@ -811,7 +809,7 @@ class ProjectedLayers:
             if ln_sink is not None:
                 return ln_sink.hand_over(dz, wp, consumer.shape)
         with dense_region("dx", hi - lo, w.size(0), w.size(1)):
-            return gemm_split(dz, self._dx_weight(layer, dz.size(1)), rows_k=False)
+            return gemm_split(dz, self._padded_weight(layer, dz.size(1)))
 
     def _padded_weight(self, layer: int, width: int) -> Tensor:
         """The layer's input projection W with zero rows up to `width` (Z's
@@ -825,22 +823,6 @@ class ProjectedLayers:
                 wp = torch.nn.functional.pad(w, (0, 0, 0, width - w.size(0)))
             self._wpad[layer] = wp
         return wp
-
-    def _dx_weight(self, layer: int, width: int) -> Tensor:
-        """The B operand of dZ W for the layer's dZ rows of `width` columns:
-        Wᵀ, with zero columns for Z's zero pad columns, formed once per epoch.
-        Whole, 16-byte aligned dZ rows take the matrix-core product; the pad
-        columns of dZ and rows of W are zero, so the sum gains only exact
-        zero terms."""
-        wt = self._wtdx.get(layer)
-        if wt is None or wt.size(1) != width:
-            w = self._proj[layer].detach()
-            with torch.no_grad():
-                if width != w.size(0):
-                    w = torch.nn.functional.pad(w, (0, 0, 0, width - w.size(0)))
-                wt = w.t().contiguous()
-            self._wtdx[layer] = wt
-        return wt
 
     def _backward_device(self, layer: int, losses: Optional[List[Tensor]] = None) -> None:
         """Backward of a projected layer: per partition, take the forward's

@@ -451,8 +451,9 @@ int gr_gemm_nt(const float* a, int64_t lda, const float* b, int64_t ldb,
                int64_t ldc, void* stream);
 
 /* gr_gemm_nt on split operands (as gr_gemm_tn): the input gradient dx = dy W
- * of the same Linear.  With b_rows_k != 0 B is [K, N] (W itself, ldb >= n) and
- * C = A B; else [N, K] as for gr_gemm_nt. */
+ * of the same Linear.  With b_rows_k != 0 B is [K, N] (W itself, ldb >= n, as
+ * this package calls it) and C = A B; else [N, K] as for gr_gemm_nt, with the
+ * same sums in the same order. */
 int gr_gemm_nt_split(const float* a, int64_t lda, const float* b, int64_t ldb,
                      int32_t b_rows_k, int64_t m, int64_t n, int64_t k, const float* bias,
                      float* c, int64_t ldc, void* stream);
