@@ -13,6 +13,13 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an AMD GPU (MI355X) and the built HIP library")
 
 
+def pytest_collection_modifyitems(items):
+    """The check that the compiled reference travelled with the tree runs
+    last: where there is no reference to build from it fails, and a run that
+    stops at its first failure has then run every other test."""
+    items.sort(key=lambda item: item.name == "test_box_compiled_reference_is_present")
+
+
 @pytest.fixture(scope="session")
 def gpu():
     """The GPU device; the HIP library must be built (no fallback exists)."""

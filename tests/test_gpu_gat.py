@@ -443,3 +443,49 @@ def test_odd_width_output_changed_in_place(gpu, C, add_bias):
         y.mul_(2.0).masked_fill_(mask, 0.0)
         torch.nn.functional.relu_(y[:, 1:])
     assert torch.equal(y, want[0])
+
+
+@pytest.mark.parametrize("H,C,offset", [(2, 4, 0), (3, 5, 0), (8, 8, 0), (8, 32, 0), (8, 27, 1),
+                                        (4, 64, 2), (2, 130, 0), (16, 64, 0), (2, 512, 0)])
+def test_several_heads_through_the_c_entries(gpu, H, C, offset):
+    """The stored-alpha entries take several heads for C callers (this package's
+    layers run those on gr_gat_heads_forward / _backward): gr_gat_forward
+    (statistics, then aggregation), gr_gat_row_dot, gr_gat_backward_src and
+    gr_gat_backward_dst against the oracle, split, empty and 16-byte unaligned
+    rows included."""
+    from grinnder_amd import _lib
+    from grinnder_amd.aggregation import _attention_backward, gat_scores
+    B, E, HC = 260, 400, H * C
+    rowptr, col, val = random_bipartite(B, E, 9, seed=H * 7 + C, long_rows=2, long_len=300)
+    adj = Adjacency(rowptr, col, val, (B, E), seg_len=64)
+    g = torch.Generator().manual_seed(H * 100 + C)
+    hs = torch.randn(E, HC, generator=g)
+    a_s, a_d = (torch.randn(1, H, C, generator=g) * C ** -0.5 for _ in range(2))
+    bias, gy = torch.randn(HC, generator=g), torch.randn(B, HC, generator=g)
+    plan = adj.device_plan(gpu)
+    f = plan.fwd
+    assert f.n_fix > 0 and plan.bwd.n_fix >= 0
+    hs_d = torch.empty(hs.numel() + offset, device=gpu)[offset:].view(hs.shape)
+    hs_d.copy_(hs)
+    s, d = gat_scores(hs_d, a_s.to(gpu), a_d.to(gpu), H, C, B)
+    m, den, cdot = (torch.full((B, H), float("nan"), device=gpu) for _ in range(3))
+    alpha = torch.full((plan.nnz, H), float("nan"), device=gpu)
+    o, y = (torch.full((B, HC), float("nan"), device=gpu) for _ in range(2))
+    b_d = bias.to(gpu)
+    ws = torch.empty(f.n_slots * ((HC + 3) // 4 * 4 + (2 * H + 3) // 4 * 4), device=gpu)
+    _lib.call("gr_gat_forward", f.units.data_ptr(), f.n_units, f.fixups.data_ptr(), f.n_fix,
+              plan.idx.data_ptr(), hs_d.data_ptr(), HC, s.data_ptr(), d.data_ptr(), B, H, C,
+              b_d.data_ptr(), m.data_ptr(), den.data_ptr(), alpha.data_ptr(), o.data_ptr(),
+              y.data_ptr(), HC, ws.data_ptr(), ws.numel(), f.n_slots, _lib.stream_handle())
+    ref, al, tpre = oracle.gat_forward(rowptr, col, hs, H, C, a_s, a_d, bias, True)
+    assert max_abs_norm_err(y, ref) <= TOL
+    assert max_abs_norm_err(o, ref - bias.double().numpy()) <= TOL
+    assert max_abs_norm_err(alpha, al) <= TOL
+    go = gy.to(gpu)
+    _lib.call("gr_gat_row_dot", go.data_ptr(), HC, o.data_ptr(), HC, B, H, C, cdot.data_ptr(),
+              _lib.stream_handle())
+    got = _attention_backward(plan, hs_d, a_s.reshape(-1).to(gpu), a_d.reshape(-1).to(gpu), s, d,
+                              alpha, den, go, cdot, H, C, False, None)
+    want = oracle.gat_backward(rowptr, col, hs, H, C, a_s, a_d, True, al, tpre, gy)
+    for a, b in zip(got, want[:3]):
+        assert max_abs_norm_err(a.reshape(-1), torch.as_tensor(b).reshape(-1)) <= TOL

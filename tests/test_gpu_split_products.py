@@ -126,6 +126,20 @@ def test_products_hold_small_and_large_magnitudes(gpu):
         assert torch.equal(got, base * 2.0 ** (e + -e // 2))
 
 
+@pytest.mark.parametrize("e", [-109, -112, -118, -125])
+def test_products_of_operands_below_the_exact_range(gpu, e):
+    """Operands below 2^-109 keep fewer than 24 bits: a bf16 piece ends at
+    2^-133, so each operand is off by at most 2^-134 and a sum over k by
+    2^-134 times the other operand's magnitudes (and its own rounding)."""
+    k = 96
+    a, b = _randn(300, k, seed=15, dev=gpu) * 2.0 ** e, _randn(70, k, seed=16, dev=gpu) * 2.0 ** 60
+    ref = a.double() @ b.double().t()
+    allowed = 2.0 ** -134 * b.double().abs().sum(1) + _bound(k) * ref.norm() / ref.numel() ** 0.5 * 8
+    assert bool(((gemm_nt_split(a, b).double() - ref).abs() <= allowed).all())
+    x, w = a.t().contiguous(), b.t().contiguous()
+    assert bool(((gemm_tn(x, w).double() - ref).abs() <= allowed).all())
+
+
 def test_products_error_and_bias_against_fp64(gpu):
     """No further from float64 than torch's fp32 product, and without the
     matrix core's bias: the mean error is far below the rms error, so sums
