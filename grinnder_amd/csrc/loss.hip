@@ -16,9 +16,10 @@
 // log_softmax + NLL; other rows are 0, or, where the train rows' bits are kept
 // for xent_backward to tell them apart, not written.
 //
-// 1M rows of 47 classes, 60% train: forward 136 us, backward 62 and four small
-// launches when every row's gradient was written, with a second exponential
-// per element, and scaled by torch; now 93 and 58 us in one launch each.
+// 1M rows of 47 classes, 60% train: forward 136 us (and 8 for the statistics'
+// last sum), backward 62 and four small launches when every row's gradient was
+// written, with a second exponential per element, and scaled by torch; now 92
+// (and 8) and 58 us, the backward in one launch.
 #include <algorithm>
 
 #include "gr_internal.h"
@@ -110,9 +111,13 @@ __device__ __forceinline__ void keep_train_bits(const uint8_t* __restrict__ mask
 // hides the loads, and few lanes with many columns each leave little of the
 // cross-lane and per-row work to a column.  1M rows of 47 classes, 60% train: a
 // row a thread with the rows staged in LDS (48 KB, three workgroups a CU)
-// 123 us, 16 lanes of 3 single columns 102 us, 4 lanes of 3 pieces 93 us (99 with
-// one step in flight).
-template <int G, int R, int V, int U>
+// 123 us, 16 lanes of 3 single columns 102 us, 4 lanes of 3 pieces 93 us.
+//
+// U is 4 while that keeps at most 48 loaded columns a lane, else 2.  Repeated
+// forward calls on 1M rows, 60% train, with 1, 2 and 4 steps (us): 10 columns
+// 31.0 / 30.6 / 30.4, 20 columns 39.8 / 39.5 / 38.9, 47 columns 78.9 / 74.5 / 72.8,
+// 60 columns 111.7 / 107.5 / 104.7, 64 columns 90.9 / 90.7 / 92.7.
+template <int G, int R, int V>
 __global__ __launch_bounds__(256) void xent_rows_narrow(const float* __restrict__ x, int64_t ld,
                                                         int64_t rows, int C,
                                                         const int64_t* __restrict__ labels,
@@ -121,7 +126,7 @@ __global__ __launch_bounds__(256) void xent_rows_narrow(const float* __restrict_
                                                         float* __restrict__ grad, int64_t ldg,
                                                         double* __restrict__ part,
                                                         uint64_t* __restrict__ bits) {
-  constexpr int RPW = 64 / G;
+  constexpr int RPW = 64 / G, U = R * V * 4 <= 48 ? 4 : 2;
   static_assert(G % U == 0, "64 rows in steps of U * RPW");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l = lane % G, sub = lane / G;
@@ -396,14 +401,14 @@ static int forward(const float* logits, int64_t ld, int64_t rows, int64_t classe
   hipStream_t s = gr::as_stream(stream);
   const int c = (int)classes;
   // With rows == 0 the single workgroup writes zero partials.
-#define GR_XENT(G, R, V, U)                                                             \
-  hipLaunchKernelGGL((xent_rows_narrow<G, R, V, U>), dim3((unsigned)nblk), dim3(256), 0, s, \
+#define GR_XENT(G, R, V)                                                                 \
+  hipLaunchKernelGGL((xent_rows_narrow<G, R, V>), dim3((unsigned)nblk), dim3(256), 0, s,   \
                      logits, ld, rows, c, labels, mask, lse, grad, ldg, workspace, bits)
-  if (c < 4) GR_XENT(4, 1, 1, 4);
-  else if (c <= 16) GR_XENT(4, 1, 4, 4);
-  else if (c <= 32) GR_XENT(4, 2, 4, 2);
-  else if (c <= 48) GR_XENT(4, 3, 4, 4);
-  else if (c <= kSmallC) GR_XENT(4, 4, 4, 1);
+  if (c < 4) GR_XENT(4, 1, 1);
+  else if (c <= 16) GR_XENT(4, 1, 4);
+  else if (c <= 32) GR_XENT(4, 2, 4);
+  else if (c <= 48) GR_XENT(4, 3, 4);
+  else if (c <= kSmallC) GR_XENT(4, 4, 4);
   else
     hipLaunchKernelGGL(xent_rows_wide, dim3((unsigned)nblk), dim3(256), 0, s, logits, ld, rows, c,
                        labels, mask, lse, grad, ldg, workspace, bits);
