@@ -599,13 +599,17 @@ def _gat_heads_ok(hs: Tensor, heads: int, channels: int) -> bool:
     """Whether the attention runs in one online-softmax pass each way
     (gr_gat_heads_forward / _backward).
 
-    Several heads: always.  One head: 36..128 channels on 16-byte rows, where the
-    one-head kernels run rows of up to 32 edges and longer ones as two launches
-    (us forward and backward / forward alone, theirs first: 48 channels over 2M
-    edges, 100k rows 327/133 and 255/102, 128 channels 447/170 and 400/155).
-    Up to 32 channels half the lanes would idle (28: 306/79 and 261/107, 176/48
-    and 246/50 for 1M edges, 30k rows), and past 128 a wavefront has one edge
-    slot either way (164: 306/121 and 338/134 there)."""
+    Several heads: always (the stored-alpha kernels with several heads serve C
+    callers only).  One head: 36..64 channels on 16-byte rows, where the one-head
+    kernels run rows of up to 32 edges and longer ones as two launches (us
+    forward and backward / forward alone, theirs first, over 100k rows: 48
+    channels, 2M edges 323/131 and 236/102, 1M edges 287/121 and 247/97; 64
+    channels 333/136 and 245/101, 299/123 and 255/98).  Up to 32 channels half
+    the lanes would idle (28: 306/79 and 261/107, 176/48 and 246/50 for 1M edges,
+    30k rows).  Past 64 a row takes half a wavefront or more either way, and
+    neither side wins over the range: 68 channels 325/116 and 297/120, but
+    266/90 and 273/102 at 1M edges; 96 channels 348/123 and 316/124, 292/95 and
+    297/103; 164 channels over 1M edges of 30k rows 281/100 and 313/112."""
     if heads == 1:
         return (channels % 4 == 0 and 32 < channels <= 64
                 and (hs.data_ptr() | 4 * hs.stride(0)) % 16 == 0)

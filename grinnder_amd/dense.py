@@ -110,8 +110,8 @@ def _row_strided(t: Tensor) -> Tensor:
 
 def gemm_split(a: Tensor, b: Tensor) -> Tensor:
     """a b for a [M, K], b [K, N]: fp32 device matrices, the operands split into
-    three bf16 pieces each (24 bits, fp32 sums; results no further from float64
-    than gemm_nt's).  The backward's products run on it; the forward's keep
+    three bf16 pieces each (24 bits, for magnitudes below 2^-109 an absolute
+    2^-134; fp32 sums; results no further from float64 than gemm_nt's).  The backward's products run on it; the forward's keep
     gemm_nt's rounding, so outputs next to an activation's kink keep their
     side."""
     _check("a", a)

@@ -425,9 +425,9 @@ int gr_xent_backward(const float* grad, int64_t rows, int64_t classes,
 /* C[M, N] = A^T B (+ beta * C) with A [K, M] (lda-strided rows) and B [K, N]
  * (ldb-strided rows), on the matrix cores with every operand split into three
  * bf16 pieces (24 bits, fp32 sums; no further from float64 than fp32 products,
- * infinities and NaN as in fp32), over `splits` chunks of K whose partial
- * tiles are summed in a fixed order (deterministic).  This
- * is the weight gradient dW = dZ^T X of the conv's dense transform (the
+ * infinities and NaN as in fp32; operands below 2^-109 in magnitude are held
+ * to 2^-134 instead), over `splits` chunks of K whose partial tiles are summed
+ * in a fixed order (deterministic).  This is the weight gradient dW = dZ^T X of the conv's dense transform (the
  * Linear inside PyG GCNConv / GATConv of grinnder/nn/gcn.py:53-56 and
  * grinnder/nn/gat.py:54-61), whose K is the partition's row count.
  * gr_gemm_tn_workspace returns the default split count and the workspace size
@@ -444,8 +444,8 @@ int gr_gemm_tn(const float* a, int64_t lda, const float* b, int64_t ldb,
  * one workgroup's sum over K (no split, deterministic).  With B = W [out, in]
  * this is the forward x W^T + b of the conv's dense transform (the Linear of
  * PyG GCNConv / GATConv, grinnder/nn/gcn.py:53-56, grinnder/nn/gat.py:54-61);
- * with B = W^T it is the input gradient dx = dy W.  bias may be NULL; m may be
- * 0 (nothing to do). */
+ * with B = W^T it is the input gradient dx = dy W in fp32 products
+ * (gr_gemm_nt_split is faster).  bias may be NULL; m may be 0 (nothing to do). */
 int gr_gemm_nt(const float* a, int64_t lda, const float* b, int64_t ldb,
                int64_t m, int64_t n, int64_t k, const float* bias, float* c,
                int64_t ldc, void* stream);
@@ -453,7 +453,9 @@ int gr_gemm_nt(const float* a, int64_t lda, const float* b, int64_t ldb,
 /* gr_gemm_nt on split operands (as gr_gemm_tn): the input gradient dx = dy W
  * of the same Linear.  With b_rows_k != 0 B is [K, N] (W itself, ldb >= n, as
  * this package calls it) and C = A B; else [N, K] as for gr_gemm_nt, with the
- * same sums in the same order. */
+ * same sums in the same order.  Rows of odd index are summed negated (against
+ * the rounding bias of the matrix core), so a row's last bits depend on its
+ * index's parity. */
 int gr_gemm_nt_split(const float* a, int64_t lda, const float* b, int64_t ldb,
                      int32_t b_rows_k, int64_t m, int64_t n, int64_t k, const float* bias,
                      float* c, int64_t ldc, void* stream);
@@ -716,7 +718,8 @@ int gr_gat_backward_dst(const int32_t* units, int64_t n_units,
  * state ([rows, H] float4) and nrow ([rows, H*C]) it also keeps what the
  * backward needs: (d, m, den, S) and N = sum of alpha Hs over the edges with
  * s + d <= 0, S the same sum of alpha.
- * Backward, from go = dL/dO and the forward's o, nrow and state: rec ([n_dst,
+ * Backward, from go = dL/dO and the forward's o, nrow and state (an infinity or
+ * NaN in one head's go stays in that head's results): rec ([n_dst,
  * H] float4, scratch), dd [n_dst, H] and ds (the gradients of d and s), and dhs
  * [rows of the plan, H*C] with both attention vectors' parts in it.
  * Workspace: n_slots times gr_gat_heads_workspace's floats (with_state != 0
