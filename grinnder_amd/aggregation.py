@@ -723,17 +723,14 @@ class _GATAttention(torch.autograd.Function):
                 keep: bool = True, trim: int = 0) -> Tensor:
         # trim: one head padded to `channels`, of which the caller wants the
         # first `trim`: the output is those columns of the padded rows, its
-        # gradient padded again.  Not a view of them, which autograd would
-        # refuse to have changed in place (views made inside a function), but
-        # a tensor of its own on their memory; so nothing saved for the
-        # backward may share that memory (gat_attention sees to it).
+        # gradient padded again.  Detached, they are no view to autograd, which
+        # refuses to have views made in here changed in place, and share the
+        # rows' version, so that such a change is found out where the rows
+        # are saved for the backward.
         y = _GATAttention._forward(ctx, hs, att_src, att_dst, bias, plan, heads, channels,
                                    concat, s_pre, d_pre, sink, zsink, zx_pre, keep)
         ctx.trim = trim
-        if not trim:
-            return y
-        return y.new_empty(0).set_(y.untyped_storage(), y.storage_offset(),
-                                   (y.size(0), trim), y.stride())
+        return y[:, :trim].detach() if trim else y
 
     @staticmethod
     def _forward(ctx, hs, att_src, att_dst, bias, plan, heads, channels, concat, s_pre, d_pre,
@@ -773,8 +770,10 @@ class _GATAttention(torch.autograd.Function):
                                                 sink)
         m = torch.empty((B, H), dtype=torch.float32, device=dev)
         den = torch.empty((B, H), dtype=torch.float32, device=dev)
-        # One head: alpha is not stored; the backward recomputes it from the
-        # destination records (gr_gat_backward_src_h1).
+        # One head (several took the one-pass kernels above): alpha is not
+        # stored; the backward recomputes it from the destination records
+        # (gr_gat_backward_src_h1), but for more than 256 channels off 16-byte
+        # alignment.
         records = _gat_records_ok(hs, H, C)
         alpha = None if records else torch.empty((max(nnz, 1), H), dtype=torch.float32,
                                                  device=dev)
@@ -1049,8 +1048,7 @@ def gat_attention(hs: Tensor, adj: Adjacency, att_src: Tensor, att_dst: Tensor,
     dHs into sink.dz at sink.rows and returns no gradient for hs.
     `trim`: a head zero-padded to `channels` returns its first `trim` (one
     head, no sink): y[:, :trim], which a caller may change in place wherever
-    it may change y; past 24 channels and with a bias its gradient is padded
-    in one launch.
+    it may change y, with the gradient padded in one launch.
     """
     _check_device_tensor("hs", hs)
     plan = adj.device_plan(hs.device)
@@ -1074,28 +1072,22 @@ def gat_attention(hs: Tensor, adj: Adjacency, att_src: Tensor, att_dst: Tensor,
                                    s, d, rowdot_sink, sink, sink.token)
     if hs.size(0) != plan.num_src:
         raise ValueError(f"hs has {hs.size(0)} rows, adjacency has {plan.num_src} columns")
-    # Outputs of up to 24 channels, and O without a bias, are saved for the
-    # backward: sliced outside the function they share the saved tensor's
-    # version, so that a change in place is seen.
-    inner = trim if bias is not None and channels > 24 else 0
     # Any input that asks for a gradient brings a backward, the scores (which
     # get none) among them.
     keep = torch.is_grad_enabled() and any(
         t is not None and t.requires_grad
         for t in (hs, att_src, att_dst, bias, *(scores or ())))
     if scores is None:
-        y = _GATAttention.apply(hs, att_src, att_dst, bias, plan, heads, channels, concat,
-                                None, None, rowdot_sink, None, None, None, keep, inner)
-        return y if inner or not trim else y[:, :trim]
+        return _GATAttention.apply(hs, att_src, att_dst, bias, plan, heads, channels, concat,
+                                   None, None, rowdot_sink, None, None, None, keep, trim)
     s, d = scores[0], scores[1]
     if tuple(s.shape) != (plan.num_src, heads) or tuple(d.shape) != (plan.num_dst, heads):
         raise ValueError("gat_attention: scores do not match the adjacency and heads")
     zx = scores[2] if len(scores) > 2 else None
     if zx is not None and tuple(zx.shape) != (plan.num_src, 32):
         raise ValueError("gat_attention: packed rows do not match the adjacency")
-    y = _GATAttention.apply(hs, att_src, att_dst, bias, plan, heads, channels, concat, s, d,
-                            rowdot_sink, None, None, zx, keep, inner)
-    return y if inner or not trim else y[:, :trim]
+    return _GATAttention.apply(hs, att_src, att_dst, bias, plan, heads, channels, concat, s, d,
+                               rowdot_sink, None, None, zx, keep, trim)
 
 
 class _GATAttentionLN(torch.autograd.Function):
